@@ -1,13 +1,13 @@
-// fp32 GEMMs on the CDNA4 matrix cores: C[M,N] (+)= op(A)[M,K] . op(B)[K,N]
-// with v_mfma_f32_16x16x4_f32.  These replace the training backward's
+// fp32 GEMMs on the CDNA4 matrix cores: C[M,N] (+)= op(A)[M,K] . op(B)[K,N],
+// small ones with v_mfma_f32_16x16x4_f32, the others as exact three-way bf16
+// splits with v_mfma_f32_32x32x16_bf16 (gemm_choice).  These replace the training backward's
 // per-position matvecs / CPU outer products:
 //   dW = dY^T X  (TN) — matmul_backward_weight_batched, pt_train.c:475-492
 //   dX = dY W    (NN) — backward_input_pretrans, pt_train.c:442-453
 //   Y  = X W^T   (NT) — the batched form of the training forward's matvecs
 //
-// Block tile TMxTN (64x64, or 32x32 for small output grids), K step 32,
-// 256 threads = 4 waves in a 2x2 grid, each wave a (TM/2)x(TN/2) sub-tile
-// of 16x16 MFMA blocks.  Tiles are staged in LDS k-major (As[k][m],
+// The small tile: 32x32, K step 32, 256 threads = 4 waves in a 2x2 grid, each
+// wave a 16x16 MFMA block.  Tiles are staged in LDS k-major (As[k][m],
 // Bs[k][n], columns XOR-swizzled so no LDS access has bank conflicts).  Two K
 // tiles are in flight in registers while a third feeds the matrix cores
 // from LDS (double-buffered), so each tile's global latency is covered by
@@ -20,6 +20,7 @@
 #include "ptmi_internal.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <utility>
@@ -29,10 +30,11 @@ namespace ptmi {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int BK = 32;
 constexpr int kXcdGrid = 768;             // grids this large take their tiles in XCD order
-constexpr int kRing64 = 2, kRing32 = 2;   // K tiles in flight per block tile size
+constexpr int kRing32 = 2;                // K tiles in flight in the 32x32 register ring
 
 struct GemmArgs {
     const float *A; long lda;
@@ -154,6 +156,55 @@ __device__ __forceinline__ void store_tile(float (*S)[R], int tid, const float (
     }
 }
 
+// Epilogue of output element (m, n) with sum v (already scaled by a fused
+// RMSNorm's 1/rms).  Columns n and n^1 of a row sit in lanes l and l^1, which
+// the fused epilogues pair with a DPP swap: every lane of a wave calls this,
+// and bounds are checked after the swap.
+template <int EPI>
+__device__ __forceinline__ void store_elem(const GemmArgs &g, float v, int m, int n, int z, float lrv) {
+    if constexpr (EPI == GEMM_EPI_ROPE) {
+        // RoPE of the q and k columns at position m (pt_ops.c:33-49;
+        // training forward pt_train.c:217)
+        const float pv = dpp_xor1(v);
+        if (n < 2 * g.epi.rope_dim) {
+            const int ip = (n < g.epi.rope_dim ? n : n - g.epi.rope_dim) & ~1;
+            float c, sn;
+            d_rope_cs(ip, g.epi.head_dim, m, &c, &sn);
+            v = (n & 1) ? pv * sn + v * c : v * c - pv * sn;
+        }
+    } else if constexpr (EPI == GEMM_EPI_SWIGLU) {
+        // columns (2i, 2i+1) = (h1, h3): out[m][i] = (h1*sigmoid(h1))*h3,
+        // the training form of silu (pt_train.c:280-284)
+        const float pv = dpp_xor1(v);
+        if (!(n & 1) && n < g.N && m < g.M) {
+            const float sig = 1.0f / (1.0f + d_expf(-v));
+            g.epi.out[(long)m * g.epi.ld + (n >> 1)] = (v * sig) * pv;
+        }
+    }
+    if (n >= g.N || m >= g.M) return;
+    if constexpr (EPI == GEMM_EPI_SWIGLU_BWD) {
+        // silu*gate backward (pt_train.c:696-721) into the interleaved
+        // (d_h1, d_h3) columns, plus silu(h1)*h3 for dW2; d_sh itself is not kept
+        const float *hp = g.epi.aux + (long)m * g.epi.aux_ld + 2 * n;
+        const float h1 = hp[0], h3 = hp[1];
+        const float sig = 1.0f / (1.0f + d_expf(-h1));
+        const float silu_val = h1 * sig;
+        g.epi.out2[(long)m * g.epi.ld2 + n] = silu_val * h3;
+        const float d_silu = v * h3;
+        float *dp = g.epi.out + (long)m * g.epi.ld + 2 * n;
+        dp[1] = v * silu_val;
+        dp[0] = d_silu * sig * (1.0f + h1 * (1.0f - sig));
+    } else if (g.partial) {
+        g.partial[((long)z * g.M + m) * g.N + n] = v;
+    } else {
+        const long o = (long)m * g.ldc + n;
+        const float cv = g.accumulate ? g.Cin[o] + v : v;
+        g.C[o] = cv;
+        // sgd_step (pt_train.c:870-873) on the weight this gradient belongs to
+        if (g.upd && !(g.keep && ((g.keep[m >> 5] >> (m & 31)) & 1u))) g.upd[o] -= lrv * cv;
+    }
+}
+
 // Epilogue of one wave's FM x FN 16x16 blocks: block (i, j) of the wave
 // covers rows mb + 16i .. and columns nb + 16j ..; lane l holds rows
 // 4*(l/16) + r, column l%16 of it (the 16x16x4 MFMA result layout).
@@ -161,9 +212,6 @@ template <int EPI, int FM, int FN>
 __device__ __forceinline__ void gemm_store(const GemmArgs &g, const floatx4 (&acc)[FM][FN], int mb, int nb, int z,
                                            int li, int lk, const float *rs = nullptr, int rs_m0 = 0) {
     const float lrv = g.upd ? *g.lr : 0.0f;
-    // C[4*(l/16)+r][l%16] of each 16x16 block; columns n and n^1 of a row sit
-    // in lanes l and l^1, which the fused epilogues pair with a DPP swap
-    // (every lane reaches it: bounds are checked after).
 #pragma unroll
     for (int i = 0; i < FM; i++) {
 #pragma unroll
@@ -174,51 +222,7 @@ __device__ __forceinline__ void gemm_store(const GemmArgs &g, const floatx4 (&ac
                 const int m = mb + i * 16 + 4 * lk + r;
                 float v = acc[i][j][r];
                 if (rs) v *= rs[m - rs_m0];                     // fused RMSNorm: the row's 1/rms
-                if constexpr (EPI == GEMM_EPI_ROPE) {
-                    // RoPE of the q and k columns at position m (pt_ops.c:33-49;
-                    // training forward pt_train.c:217)
-                    const float pv = dpp_xor1(v);
-                    if (n < 2 * g.epi.rope_dim) {
-                        const int ip = (n < g.epi.rope_dim ? n : n - g.epi.rope_dim) & ~1;
-                        float c, sn;
-                        d_rope_cs(ip, g.epi.head_dim, m, &c, &sn);
-                        v = (n & 1) ? pv * sn + v * c : v * c - pv * sn;
-                    }
-                } else if constexpr (EPI == GEMM_EPI_SWIGLU) {
-                    // columns (2i, 2i+1) = (h1, h3): out[m][i] = (h1*sigmoid(h1))*h3,
-                    // the training form of silu (pt_train.c:280-284)
-                    const float pv = dpp_xor1(v);
-                    if (!(n & 1) && n < g.N && m < g.M) {
-                        const float sig = 1.0f / (1.0f + d_expf(-v));
-                        g.epi.out[(long)m * g.epi.ld + (n >> 1)] = (v * sig) * pv;
-                    }
-                }
-                if constexpr (EPI == GEMM_EPI_SWIGLU_BWD) {
-                    // silu*gate backward (pt_train.c:696-721) into the interleaved
-                    // (d_h1, d_h3) columns, plus silu(h1)*h3 for dW2
-                    if (n < g.N && m < g.M) {
-                        const float *hp = g.epi.aux + (long)m * g.epi.aux_ld + 2 * n;
-                        const float h1 = hp[0], h3 = hp[1];
-                        const float sig = 1.0f / (1.0f + d_expf(-h1));
-                        const float silu_val = h1 * sig;
-                        g.epi.out2[(long)m * g.epi.ld2 + n] = silu_val * h3;
-                        const float d_silu = v * h3;
-                        float *dp = g.epi.out + (long)m * g.epi.ld + 2 * n;
-                        dp[1] = v * silu_val;
-                        dp[0] = d_silu * sig * (1.0f + h1 * (1.0f - sig));
-                    }
-                    continue;                                   // d_sh itself is not kept
-                }
-                if (n >= g.N || m >= g.M) continue;
-                if (g.partial) {
-                    g.partial[((long)z * g.M + m) * g.N + n] = v;
-                } else {
-                    const long o = (long)m * g.ldc + n;
-                    const float cv = g.accumulate ? g.Cin[o] + v : v;
-                    g.C[o] = cv;
-                    // sgd_step (pt_train.c:870-873) on the weight this gradient belongs to
-                    if (g.upd && !(g.keep && ((g.keep[m >> 5] >> (m & 31)) & 1u))) g.upd[o] -= lrv * cv;
-                }
+                store_elem<EPI>(g, v, m, n, z, lrv);
             }
         }
     }
@@ -456,18 +460,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
 // step s -> k = 4g + s), so every product pairs the same k.
 // Two LDS stages: the loads of tile s+1 are issued before the MFMAs of tile
 // s and waited for (vmcnt, in order) at the next step's barrier.
-// The classifier's weight gradient (TN) runs on these tiles, its forward
-// (NT) on the 32x32x2 form below (gemm_tile_dl32).
-// Measured on the MI355X against the register-ring kernel (launches back to
-// back, same inputs, same bits): NT 256x32000x288 with 256x128 tiles, 47.2
-// vs 51.3 us; TN 32000x288x255 with 64x96 tiles, 55.5 vs 58.7 us, and with
-// 128x96 tiles on 8 waves (4x2) 51.1-52.9 vs 53.6-55.1 us (graph-replayed,
-// same output bits; 128x96 on 4 or 8x1 waves, 256x96, 64x96 on 8 waves,
-// 64x288 and 128x288 were slower).  NT 256x128 on 8x1 or 2x4 waves and
-// 256x64 tiles were no faster than 4x2.  Deeper
-// stage rings, 64-k stages, and loads interleaved one per MFMA k step were
-// all slower; so were these tiles on the per-layer shapes (5-16 us against
-// 5-10 us) and on the long-K NN (split K, 68 vs 60 us).
+// Large weight gradients (TN) over fewer than 256 positions run on these
+// tiles; longer ones and the classifier's forward (NT) take the bf16-product
+// tiles below.  Measured on the MI355X against the register-ring kernel: TN
+// 32000x288x255 with 64x96 tiles 55.5 vs 58.7 us, and with 128x96 tiles on 8
+// waves (4x2) 51.1-52.9 vs 53.6-55.1 us (graph-replayed, same output bits;
+// 128x96 on 4 or 8x1 waves, 256x96, 64x96 on 8 waves, 64x288 and 128x288 were
+// slower).  Deeper stage rings, 64-k stages, and loads interleaved one per
+// MFMA k step were all slower.
 constexpr int kDlStages = 2;
 
 // Chunk-slot swizzle of row i of a k-contiguous tile: i & 7 spreads 8
@@ -677,142 +677,424 @@ __device__ __forceinline__ void gemm_tile_panel(const GemmArgs &g, int m0, int n
     gemm_store<EPI, 1, 1>(g, acc, m0 + wm * 16, n0 + wn * 16, z, li, lk);
 }
 
-// The NT direct-to-LDS tile on v_mfma_f32_32x32x2_f32 (the classifier's
-// forward: both operands k-contiguous, same LDS layout and DMA loads as
-// gemm_tile_dl).  In 8-k block q, lane half h = l/32 of a 32-lane group
-// reads chunk 2q + h of its row as one b128, so step s pairs k = 8q + s
-// (h = 0) with k = 8q + 4 + s (h = 1); A and B use the same order.  The 8
-// lanes of a b128 access phase hit 8 distinct chunk slots, as in
-// gemm_tile_dl.  C[(v/4)*8 + 4h + v%4][l%32] is component v of the lane's
-// 16 sums; the tile goes out through LDS as whole rows, a float4 per lane.
-// Measured on the MI355X for the 15M classifier (256 x 32000 x 288,
-// interleaved launches): 44.5-49.9 us against 45.7-51.4 us for the 16x16x4
-// tile, the same bits on integer-valued operands.  Four waves per SIMD
-// (16-wave 256x128 tiles, or two 128x128 workgroups per CU) and a third LDS
-// stage gave no further gain: each 32-k step costs ~4.0 us in every form,
-// the rate of one wave's MFMA issue.
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-template <int TM, int TN, int WM, int WN>
-__device__ __forceinline__ void gemm_tile_dl32(const GemmArgs &g, int m0, int n0, int z) {
-    constexpr int NW = WM * WN, NS = kDlStages, CPI = BK / 4;
-    constexpr int FM = TM / WM / 32, FN = TN / WN / 32;
-    static_assert(FM * WM * 32 == TM && FN * WN * 32 == TN, "tile");
-    constexpr int STAGE = (TM + TN) * BK;
-    __shared__ __align__(16) float smem[NS * STAGE + 256];
-    float *junk = smem + NS * STAGE;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WN, wn = wave % WN;
-    const int li = lane & 31, lh = lane >> 5;
-    const int kb = z * g.k_per_split;
-    const int kend = min(g.K, kb + g.k_per_split);
+// ── fp32 products on the bf16 matrix cores ───────────────────────────────
+// The large and middle GEMMs.  v_mfma_f32_32x32x16_bf16 runs 16x the
+// multiply-adds per cycle of v_mfma_f32_32x32x2_f32, and an fp32 number is
+// exactly the sum of three bf16: x = h + m + l, h the nearest bf16, m the top
+// 8 bits of x - h, l the rest (24 significant bits in all).  a*b is taken as
+// the six largest of the nine partial products, smallest first into one fp32
+// accumulator: al*bh, ah*bl, am*bm, am*bh, ah*bm, ah*bh.  The three dropped are below
+// 2^-24 of |a*b| and of either sign (h is rounded, not cut), and the
+// accumulator rounds 6 times per 16 k instead of 16 times, so results are
+// nearer to 64-bit sums than the fp32 MFMA tiles' (relative error at K = 768
+// and 2048: 5.0e-7 and 8.1e-7 before, 4.2e-7 and 6.9e-7 in 128x128 tiles,
+// 2.1e-7 and 3.4e-7 in 64x64 tiles, whose four waves each sum a quarter of
+// K).  Numbers below 2^-109 lose low bits (bf16 reaches down to 2^-133).  A
+// tile with a non-finite sum is computed again with fp32 MFMAs, so
+// infinities, NaNs and numbers that round past the bf16 range come out as
+// the fp32 tiles give them.
+// What bounds it: the MFMAs (32 cycles each) and the splits (7 VALU
+// instructions per MFMA) issue side by side; with the splits taken out the same
+// kernels reach 180-195 TFLOP/s, the bf16 matrix rate under the card's power limit.
+//
+// Operand tiles reach LDS as fp32 by DMA, KD = 16 or 32 k at a time, in whole
+// 16-byte chunks: k-contiguous operands as rows of KD floats with the chunks
+// of row i permuted so that 16 rows' same chunk spread over all banks;
+// k-major operands as rows of TI floats with bit 5 of the column flipped
+// where bit 3 of k is set (a lane half reads 8 k, the other half the next 8).
+// The loads are buffer loads with a per-lane offset: elements outside the
+// operand get an offset past the descriptor's range and come back as zeros,
+// so addresses are worked out once per tile (again for a ragged K step) and
+// no load is under a branch.  E floats per lane and load: 4, or 1 where rows
+// are not 16-byte aligned (the same tile with four times the load
+// instructions: NT 1024x2048x768 24.9 -> 28.3 us).
+constexpr int kOutside = (int)0x80000000;     // past every descriptor's range
+
+// 16 or 4 bytes per lane to lds + lane * size.
+typedef void __attribute__((address_space(3))) *lds_ptr;
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, float *lds, int off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)lds, 16, off, 0, 0, 0);
+}
+__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t rs, float *lds, int off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)lds, 4, off, 0, 0, 0);
+}
+
+template <bool KMAJOR, int TI, int KD, int E, int NW>
+struct TileDma {
+    static constexpr int N = TI * KD / (64 * E * NW);           // loads per wave
+    static_assert(N * 64 * E * NW == TI * KD && (KD == 16 || KD == 32), "whole loads");
+    int off[N];
+    static __device__ __forceinline__ int swz(int i) { return KD == 32 ? kc_swz(i) : (i >> 2) & 3; }
+    // This lane's byte offsets from the tile's first element; krem: the k
+    // left from there.  ld < kMaxSplitLd keeps them below 2^31.
+    __device__ __forceinline__ void init(long ld, int ilim, int i0, int wave, int lane, int krem) {
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const int S = E * ((j * NW + wave) * 64 + lane);    // position in the tile
+            int i, k;
+            if constexpr (KMAJOR) {
+                k = S / TI;
+                i = (S % TI) ^ (((k >> 3) & 1) << 5);
+            } else {
+                i = S / KD;
+                k = 4 * (((S % KD) >> 2) ^ swz(i)) + (S & 3);
+            }
+            const long o = KMAJOR ? (long)k * ld + i : (long)i * ld + k;
+            off[j] = i0 + i < ilim && k < krem ? (int)(4 * o) : kOutside;
+        }
+    }
+    // records: 0x7fffffff, or 0 to load zeros only
+    __device__ __forceinline__ void issue(const float *base, int records, float *lds, int wave) const {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, records, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            float *dst = lds + (j * NW + wave) * 64 * E;
+            if constexpr (E == 4) dma16(rs, dst, off[j]);
+            else dma4(rs, dst, off[j]);
+        }
+    }
+    // x[e] = element (i, k = 16q + 8*lh + e) of the tile in LDS
+    static __device__ __forceinline__ void read(const float *t, int i, int q, int lh, float (&x)[8]) {
+        if constexpr (KMAJOR) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = t[(16 * q + 8 * lh + e) * TI + (i ^ (lh << 5))];
+        } else {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const floatx4 v = *reinterpret_cast<const floatx4 *>(t + i * KD + 4 * ((4 * q + 2 * lh + c) ^ swz(i)));
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[4 * c + e] = v[e];
+            }
+        }
+    }
+};
+constexpr long kMaxSplitLd = 1L << 22;        // 127 rows of it stay below 2^31 bytes
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+// x[e] = o[0][e] + o[1][e] + o[2][e] (see above).
+__device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&o)[3]) {
+    constexpr unsigned kTop = 0xffff0000u, kHighHalves = 0x07060302u;
+    uintx4 h, m, l;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const floatx2 v = {x[2 * e], x[2 * e + 1]};
+        h[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+        const float r0 = v.x - __uint_as_float(h[e] << 16), r1 = v.y - __uint_as_float(h[e] & kTop);
+        const unsigned u0 = __float_as_uint(r0), u1 = __float_as_uint(r1);
+        const float l0 = r0 - __uint_as_float(u0 & kTop), l1 = r1 - __uint_as_float(u1 & kTop);
+        m[e] = __builtin_amdgcn_perm(u1, u0, kHighHalves);
+        l[e] = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), kHighHalves);
+    }
+    o[0] = __builtin_bit_cast(bf16x8, h);
+    o[1] = __builtin_bit_cast(bf16x8, m);
+    o[2] = __builtin_bit_cast(bf16x8, l);
+}
+
+// Two 32-row fragments of each operand: 16 k in fp32, and split.
+struct RawFrags { float a[2][8], b[2][8]; };
+struct SplitFrags { bf16x8 a[2][3], b[2][3]; };
+
+__device__ __forceinline__ void split_frags(const RawFrags &x, SplitFrags &o) {
+#pragma unroll
+    for (int f = 0; f < 2; f++) split_bf16(x.a[f], o.a[f]);
+#pragma unroll
+    for (int f = 0; f < 2; f++) split_bf16(x.b[f], o.b[f]);
+}
+
+__device__ __forceinline__ void split_products(const SplitFrags &x, floatx16 (&acc)[2][2]) {
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int p = 0; p < 6; p++)
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                acc[f][h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.a[f][pa[p]], x.b[h][pb[p]], acc[f][h], 0, 0, 0);
+}
+
+template <int F>
+__device__ __forceinline__ void zero_acc(floatx16 (&acc)[F][F]) {
+#pragma unroll
+    for (int f = 0; f < F; f++)
+#pragma unroll
+        for (int h = 0; h < F; h++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[f][h][v] = 0.0f;
+}
+
+// This wave's loads have landed (vmcnt) and its LDS reads are done (lgkmcnt:
+// their values may be used only later).
+__device__ __forceinline__ void wait_loads_and_reads() {
+    __builtin_amdgcn_s_waitcnt(7 << 4);                         // vmcnt(0) lgkmcnt(0)
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void wait_reads() {
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));      // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+}
+// The same for every wave of the block.
+__device__ __forceinline__ void block_loads_and_reads() {
+    wait_loads_and_reads();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// The T x T tile at (m0, n0) over k in [kb, kend) with fp32 MFMAs, on 2 x 2
+// waves of T/2 x T/2: the non-finite case above.  smem: 4*T*BK floats.
+template <bool AK, bool BKM, int T, int E>
+__device__ __forceinline__ void fp32_mma(const GemmArgs &g, int m0, int n0, int kb, int kend, float *smem,
+                                         floatx16 (&acc)[T / 64][T / 64]) {
+    constexpr int F = T / 64, STAGE = 2 * T * BK;
+    using DA = TileDma<AK, T, BK, E, 4>;
+    using DB = TileDma<BKM, T, BK, E, 4>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1, li = lane & 31, lh = lane >> 5;
+    zero_acc<F>(acc);
+    for (int k0 = kb; k0 < kend; k0 += BK) {
+        DA da;
+        DB db;
+        da.init(g.lda, g.M, m0, wave, lane, kend - k0);
+        db.init(g.ldb, g.N, n0, wave, lane, kend - k0);
+        da.issue(g.A + (AK ? (long)k0 * g.lda + m0 : (long)m0 * g.lda + k0), 0x7fffffff, smem, wave);
+        db.issue(g.B + (BKM ? (long)k0 * g.ldb + n0 : (long)n0 * g.ldb + k0), 0x7fffffff, smem + T * BK, wave);
+        block_loads_and_reads();
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            float xa[F][8], xb[F][8];
+#pragma unroll
+            for (int f = 0; f < F; f++) {
+                DA::read(smem, wm * (T / 2) + f * 32 + li, q, lh, xa[f]);
+                DB::read(smem + T * BK, wn * (T / 2) + f * 32 + li, q, lh, xb[f]);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+#pragma unroll
+                for (int f = 0; f < F; f++)
+#pragma unroll
+                    for (int h = 0; h < F; h++)
+                        acc[f][h] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[f][e], xb[h][e], acc[f][h], 0, 0, 0);
+        }
+        block_loads_and_reads();
+    }
+    static_assert(STAGE <= 4 * T * BK, "one stage");
+}
+
+// 128x128 output tile at (m0, n0) over K range split z: 2 x 2 waves of
+// 64x64, K steps of 32 in two LDS stages.  A wave's splits of one 16-k block
+// go between its MFMAs of the block before; the next tile's loads are in
+// flight meanwhile.  For outputs of many tiles and short K (gemm_split_tile), where
+// the 64x64 tile's start and sum cost more than its lighter splits save: NT
+// 1024x32000x768 474 -> 340 us (64x64 tiles 396), TN 32000x768x1024 528 -> 340.
+template <bool AK, bool BKM, int E, int EPI>
+__device__ __forceinline__ void gemm_tile_split128(const GemmArgs &g, int m0, int n0, int z) {
+    constexpr int T = 128, STAGE = 2 * T * BK;
+    using DA = TileDma<AK, T, BK, E, 4>;
+    using DB = TileDma<BKM, T, BK, E, 4>;
+    __shared__ __align__(16) float smem[2 * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1, li = lane & 31, lh = lane >> 5;
+    const int kb = z * g.k_per_split, kend = min(g.K, kb + g.k_per_split);
     const int nk = kb < kend ? (kend - kb + BK - 1) / BK : 0;
-
-    floatx16 acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
-
-    auto issue = [&](int t) {
-        float *st = smem + (t % NS) * STAGE;
-        const int k0 = kb + t * BK;
-        dl_issue<false, TM, NW>(g.A, g.lda, g.M, m0, k0, kend, st, junk, wave, lane);
-        dl_issue<false, TN, NW>(g.B, g.ldb, g.N, n0, k0, kend, st + TM * BK, junk, wave, lane);
+    const float *A0 = g.A + (AK ? (long)kb * g.lda + m0 : (long)m0 * g.lda + kb);
+    const float *B0 = g.B + (BKM ? (long)kb * g.ldb + n0 : (long)n0 * g.ldb + kb);
+    const long stepA = AK ? BK * g.lda : BK, stepB = BKM ? BK * g.ldb : BK;
+    DA da;
+    DB db;
+    auto place = [&](int krem) {
+        da.init(g.lda, g.M, m0, wave, lane, krem);
+        db.init(g.ldb, g.N, n0, wave, lane, krem);
     };
-    // row i of a k-contiguous tile, k = 8q + 4h + s in component s
-    auto rd = [&](const float *base, int i, int q) {
-        return *reinterpret_cast<const floatx4 *>(base + (i * CPI + ((2 * q + lh) ^ kc_swz(i))) * 4);
+    auto issue = [&](int s) {
+        if (s == nk - 1 && s > 0) place(kend - kb - s * BK);    // the last K step may be ragged
+        float *st = smem + (s & 1) * STAGE;
+        da.issue(A0 + s * stepA, 0x7fffffff, st, wave);
+        db.issue(B0 + s * stepB, 0x7fffffff, st + T * BK, wave);
     };
-
-    if (nk > 0) issue(0);
-    for (int s = 0; s < nk; s++) {
-        // as gemm_tile_dl: tile s is in once this wave's loads are done and
-        // every wave is past the barrier, which also ends the reads of the
-        // stage that tile s+1 overwrites
-        wait_vmcnt<0>();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (s + 1 < nk) issue(s + 1);
-        const float *st = smem + (s % NS) * STAGE, *sb = st + TM * BK;
-        floatx4 a[4][FM], b[4][FN];
+    RawFrags x;
+    auto read = [&](int s, int q) {
+        const float *st = smem + (s & 1) * STAGE;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int f = 0; f < 2; f++) DA::read(st, wm * 64 + f * 32 + li, q, lh, x.a[f]);
 #pragma unroll
-            for (int f = 0; f < FM; f++) a[q][f] = rd(st, wm * (TM / WM) + f * 32 + li, q);
-#pragma unroll
-            for (int h = 0; h < FN; h++) b[q][h] = rd(sb, wn * (TN / WN) + h * 32 + li, q);
+        for (int f = 0; f < 2; f++) DB::read(st + T * BK, wn * 64 + f * 32 + li, q, lh, x.b[f]);
+    };
+    floatx16 acc[2][2];
+    zero_acc<2>(acc);
+    if (nk > 0) {                                               // uniform
+        SplitFrags s0, s1;
+        place(min(BK, kend - kb));
+        issue(0);
+        block_loads_and_reads();
+        if (nk > 1) issue(1);
+        read(0, 0);
+        split_frags(x, s0);
+        for (int s = 0; s < nk; s++) {
+            read(s, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            split_products(s0, acc);
+            split_frags(x, s1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + 1 < nk) {
+                // tile s+1 is in, and every wave has read tile s, whose
+                // stage tile s+2 overwrites
+                block_loads_and_reads();
+                if (s + 2 < nk) issue(s + 2);
+                read(s + 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            split_products(s1, acc);
+            split_frags(x, s0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-#pragma unroll
-            for (int ss = 0; ss < 4; ss++)
-#pragma unroll
-                for (int f = 0; f < FM; f++)
-#pragma unroll
-                    for (int h = 0; h < FN; h++)
-                        acc[f][h] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][f][ss], b[q][h][ss], acc[f][h], 0, 0, 0);
     }
-    // C, or this split's partial product (partial + z*M*N, ld N)
-    const int mb = m0 + wm * (TM / WM), nb = n0 + wn * (TN / WN);
-    const bool part = g.partial != nullptr, accum = !part && g.accumulate;
-    float *const out = part ? g.partial + (long)z * g.M * g.N : g.C;
-    const long ldo = part ? (long)g.N : g.ldc;
-    if (!(ldo & 3) && !((uintptr_t)out & 15) && (!accum || !((uintptr_t)g.Cin & 15))) {
-        // Each wave stages RP rows x W columns at a time in its own LDS
-        // region (the stage buffers are free once every wave is past the
-        // loop) and stores whole rows, a float4 per lane.
-        constexpr int W = FN * 32, P = W + 4, RP = NW * 32 * P <= NS * STAGE ? 32 : 16;
-        static_assert(NW * RP * P <= NS * STAGE, "store staging");
+    bool finite = true;
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) finite = finite && fabsf(acc[f][h][v]) <= 3.4028235e+38f;
+    if (__syncthreads_or(!finite)) fp32_mma<AK, BKM, T, E>(g, m0, n0, kb, kend, smem, acc);     // uniform
+    // C[(v/4)*8 + 4*(l/32) + v%4][l%32] is component v of lane l
+    const int mb = m0 + wm * 64 + 4 * lh, nb = n0 + wn * 64 + li;
+    const float lrv = g.upd ? *g.lr : 0.0f;
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                store_elem<EPI>(g, acc[f][h][v], mb + f * 32 + (v >> 2) * 8 + (v & 3), nb + h * 32, z, lrv);
+}
+
+// 64x64 output tile at (m0, n0) over K range split z, K dealt to the four waves:
+// wave w takes the 16-k blocks w, w+4, ... of the whole tile, through two LDS
+// stages of its own, and the four sums meet in LDS at the end.  So no barrier
+// lies in the main loop, every element is split once per block (2 x 2 waves
+// of 32x32 split each twice), and a lone block per CU keeps all four SIMDs
+// on MFMAs with independent accumulators (as 2 x 2 waves a K step of 32
+// takes 0.65-0.85 us there, here about 0.25).  A ragged last block comes first in
+// its wave's order, so its offsets cost one more init and no extra wait.
+// Measured (launches back to back; the 32x32 and 64x64 fp32 tiles before):
+// NT 1024x2048x768 41.6 -> 24.9 us, NN 1024x768x2048 45.7 -> 27.1, TN
+// 2048x768x1024 43.2 -> 27.0, NN 1024x768x32000 562 -> 291.  Three or four
+// stages (one block per CU) and eight waves were slower except for a lone
+// block per CU (27.1 -> 25.4 with eight waves).
+template <bool AK, bool BKM, int E, int EPI>
+__device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int n0, int z) {
+    constexpr int T = 64, KD = 16, NS = 2, NW = 4, STAGE = 2 * T * KD;
+    using DA = TileDma<AK, T, KD, E, 1>;
+    using DB = TileDma<BKM, T, KD, E, 1>;
+    constexpr int LPT = DA::N + DB::N;
+    static_assert((NS - 1) * LPT < 64, "vmcnt");
+    __shared__ __align__(16) float smem[NW * NS * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int kb = z * g.k_per_split, kend = min(g.K, kb + g.k_per_split);
+    const int nf = max(0, kend - kb) / KD, tail = max(0, kend - kb) % KD;     // whole blocks, ragged k
+    const int first = tail > 0 && nf % NW == wave;               // 1: the ragged block is this wave's block 0
+    const int n = first + (nf - wave + NW - 1) / NW;
+    const float *A0 = g.A + (AK ? (long)kb * g.lda + m0 : (long)m0 * g.lda + kb);
+    const float *B0 = g.B + (BKM ? (long)kb * g.ldb + n0 : (long)n0 * g.ldb + kb);
+    const long stepA = AK ? KD * g.lda : KD, stepB = BKM ? KD * g.ldb : KD;
+    float *ring = smem + wave * NS * STAGE;
+    DA da;
+    DB db;
+    auto place = [&](int krem) {
+        da.init(g.lda, g.M, m0, 0, lane, krem);
+        db.init(g.ldb, g.N, n0, 0, lane, krem);
+    };
+    // this wave's block j (past its last: zeros) into its stage `st`
+    auto issue = [&](int j, int st) {
+        const bool in = j < n;
+        const long c = !in ? 0 : first && j == 0 ? nf : (long)(j - first) * NW + wave;
+        float *d = ring + st * STAGE;
+        da.issue(A0 + c * stepA, in ? 0x7fffffff : 0, d, 0);
+        db.issue(B0 + c * stepB, in ? 0x7fffffff : 0, d + T * KD, 0);
+    };
+    RawFrags x;
+    auto read = [&](int st) {
+        const float *p = ring + st * STAGE;
+#pragma unroll
+        for (int f = 0; f < 2; f++) DA::read(p, f * 32 + li, 0, lh, x.a[f]);
+#pragma unroll
+        for (int f = 0; f < 2; f++) DB::read(p + T * KD, f * 32 + li, 0, lh, x.b[f]);
+    };
+    floatx16 acc[2][2];
+    zero_acc<2>(acc);
+    if (n > 0) {                                                // wave-uniform
+        SplitFrags s0, s1;
+        if (first) place(tail);
+        else place(KD);
+        issue(0, 0);
+        if (first) place(KD);
+        issue(1, 1);
+        wait_vmcnt<LPT>();
+        asm volatile("" ::: "memory");
+        read(0);
+        split_frags(x, s0);
+        wait_reads();
+        issue(2, 0);
+        for (int j = 0; j < n; j += 2) {
+            // blocks j+1 and j+2 are in flight, s0 holds block j's parts
+            wait_vmcnt<LPT>();
+            asm volatile("" ::: "memory");
+            read(1);
+            __builtin_amdgcn_sched_barrier(0);
+            split_products(s0, acc);
+            split_frags(x, s1);
+            __builtin_amdgcn_sched_barrier(0);
+            wait_reads();
+            issue(j + 3, 1);
+            wait_vmcnt<LPT>();
+            asm volatile("" ::: "memory");
+            read(0);
+            __builtin_amdgcn_sched_barrier(0);
+            split_products(s1, acc);
+            split_frags(x, s0);
+            __builtin_amdgcn_sched_barrier(0);
+            wait_reads();
+            issue(j + 4, 0);
+        }
+    }
+    block_loads_and_reads();                                    // the rings are free
+    // C[(v/4)*8 + 4*lh + v%4][l%32] is component v; columns of rows with bit
+    // 2 set are flipped by 32 (the two lane halves then use different banks)
+    float *const red = smem;
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                red[(wave * T + f * 32 + (v >> 2) * 8 + 4 * lh + (v & 3)) * T + ((h * 32 + li) ^ (lh << 5))] = acc[f][h][v];
+    __syncthreads();
+    // wave w sums rows w, w+4, ...; lane = column
+    float sum[T / NW];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < T / NW; e++) {
+        const float *p = red + (e * NW + wave) * T + (lane ^ ((e & 1) << 5));      // row bit 2 = bit 0 of e
+        sum[e] = ((p[0] + p[T * T]) + p[2 * T * T]) + p[3 * T * T];
+        finite = finite && fabsf(sum[e]) <= 3.4028235e+38f;
+    }
+    if (__syncthreads_or(!finite)) {                            // uniform
+        floatx16 fa[1][1];
+        fp32_mma<AK, BKM, T, E>(g, m0, n0, kb, kend, smem, fa);
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            red[((wave >> 1) * 32 + (v >> 2) * 8 + 4 * lh + (v & 3)) * T + (wave & 1) * 32 + li] = fa[0][0][v];
         __syncthreads();
-        float *T = smem + wave * RP * P;
 #pragma unroll
-        for (int f = 0; f < FM; f++) {
-#pragma unroll
-            for (int p = 0; p < 32 / RP; p++) {
-                // components v of rows [p*RP, p*RP + RP) (a wave's LDS
-                // operations complete in order, so this pass's reads are
-                // done before the next pass overwrites the region)
-#pragma unroll
-                for (int h = 0; h < FN; h++)
-#pragma unroll
-                    for (int v = p * RP / 2; v < (p + 1) * RP / 2; v++)
-                        T[((v >> 2) * 8 + 4 * lh + (v & 3) - p * RP) * P + h * 32 + li] = acc[f][h][v];
-                for (int e4 = lane; e4 < RP * W / 4; e4 += 64) {
-                    const int r = e4 / (W / 4), c = 4 * (e4 % (W / 4));
-                    const floatx4 val = *reinterpret_cast<const floatx4 *>(T + r * P + c);
-                    const int m = mb + f * 32 + p * RP + r, n = nb + c;
-                    if (m >= g.M) continue;
-                    const long o = (long)m * ldo + n;
-                    if (n + 3 < g.N) {
-                        floatx4 cv = val;
-                        if (accum) cv += *reinterpret_cast<const floatx4 *>(g.Cin + o);
-                        *reinterpret_cast<floatx4 *>(out + o) = cv;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (n + e < g.N) out[o + e] = accum ? g.Cin[o + e] + val[e] : val[e];
-                    }
-                }
-            }
-        }
-        return;
+        for (int e = 0; e < T / NW; e++) sum[e] = red[(e * NW + wave) * T + lane];
     }
+    const float lrv = g.upd ? *g.lr : 0.0f;
 #pragma unroll
-    for (int f = 0; f < FM; f++)
-#pragma unroll
-        for (int h = 0; h < FN; h++) {
-            const int n = nb + h * 32 + li;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m = mb + f * 32 + (v >> 2) * 8 + 4 * lh + (v & 3);
-                if (n >= g.N || m >= g.M) continue;
-                const long o = (long)m * ldo + n;
-                out[o] = accum ? g.Cin[o] + acc[f][h][v] : acc[f][h][v];
-            }
-        }
+    for (int e = 0; e < T / NW; e++) store_elem<EPI>(g, sum[e], m0 + e * NW + wave, n0 + lane, z, lrv);
 }
 
 // Workgroups go to the 8 XCDs round-robin by linear id, and each XCD has its
@@ -857,21 +1139,6 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_dl(GemmArgs g) {
     gemm_tile_dl<AK, BKM, TM, TN, WM, WN>(g, m * TM, n * TN, z);
 }
 
-// The classifier's NT forward on the 32x32x2 tiles (grid and tile order as k_gemm).
-template <int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN) void k_gemm_dl32(GemmArgs g) {
-    const int gx = gridDim.x, gy = gridDim.y, per_z = gx * gy, total = per_z * gridDim.z;
-    int m = blockIdx.y, n = blockIdx.x, z = blockIdx.z;
-    if (total >= kXcdGrid) {                                        // uniform
-        const int t = xcd_tile(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), total);
-        z = t / per_z;
-        const int u = t - z * per_z;
-        if (g.M > g.N) m = u / gx, n = u - m * gx;
-        else n = u / gy, m = u - n * gy;
-    }
-    gemm_tile_dl32<TM, TN, WM, WN>(g, m * TM, n * TN, z);
-}
-
 // The per-layer panel GEMM (grid and tile order as k_gemm).
 template <bool BKM, int NSK, int EPI>
 __global__ __launch_bounds__(256) void k_gemm_panel(GemmArgs g) {
@@ -885,6 +1152,19 @@ __global__ __launch_bounds__(256) void k_gemm_panel(GemmArgs g) {
         else n = u / gy, m = u - n * gy;
     }
     gemm_tile_panel<BKM, NSK, EPI>(g, m * 32, n * 32, z);
+}
+
+// The bf16-product GEMMs (grid of T x T tiles, T = 64 or 128; tile order as k_gemm).
+template <bool AK, bool BKM, int T, int E, int EPI>
+__global__ __launch_bounds__(256, 2) void k_gemm_split(GemmArgs g) {
+    const int gx = gridDim.x, gy = gridDim.y, per_z = gx * gy, total = per_z * gridDim.z;
+    const int t = xcd_tile(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), total);
+    const int z = t / per_z, u = t - z * per_z;
+    int m, n;
+    if (g.M > g.N) m = u / gx, n = u - m * gx;
+    else n = u / gy, m = u - n * gy;
+    if constexpr (T == 128) gemm_tile_split128<AK, BKM, E, EPI>(g, m * T, n * T, z);
+    else gemm_tile_slice64<AK, BKM, E, EPI>(g, m * T, n * T, z);
 }
 
 // Grouped TN GEMMs (32x32 tiles, whole K): block b runs tile
@@ -916,14 +1196,17 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float *partial, int
 
 inline bool al16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-bool gemm_big_tiles(int op, int M, int N, int K) { return K >= 4096 || (op == 2 && (long)M * N >= (4L << 20)); }
+constexpr size_t kScratchFloats = (size_t)4 << 20;      // split-K partials of ptmi_gemm_dev_noalloc
 
-// How launch_gemm splits K: `chosen` splits fit the workspace, then K is
-// cut into whole K steps per split, which gives `splits` (<= chosen).
+// How many splits the fp32 tiles take: 32x32 tiles with K cut into whole
+// steps of at least eight per split where the grid is small.  K >= 4096 counts
+// 64x64 tiles and splits to 1024 blocks (the count ptmi_gemm_dev_noalloc
+// admits calls by, and the one split sums are held against).  `chosen` splits
+// fit the workspace; cutting K into whole steps gives `splits` (<= chosen).
 struct SplitPlan { int chosen, splits, k_per_split; };
 SplitPlan split_plan(int op, int M, int N, int K, size_t ws_floats, int ek) {
     if (ek != GEMM_EPI_NONE) return SplitPlan{1, 1, K};          // the epilogue needs whole-K sums
-    const bool big = gemm_big_tiles(op, M, N, K);
+    const bool big = K >= 4096 || (op == 2 && (long)M * N >= (4L << 20));
     const int T = big ? 64 : 32;
     const long blocks = (long)((N + T - 1) / T) * ((M + T - 1) / T);
     const int nk = (K + BK - 1) / BK;
@@ -936,14 +1219,68 @@ SplitPlan split_plan(int op, int M, int N, int K, size_t ws_floats, int ek) {
     return SplitPlan{chosen, (K + kps - 1) / kps, kps};
 }
 
+// Tile and K split of a GEMM: 32 (fp32 MFMA tiles, `splits` from split_plan),
+// 64 or 128 (bf16 products).  The smallest estimate of the launch's time in
+// µs, fitted to launches back to back on the MI355X (256 CUs; n = blocks per
+// CU, measured -> estimated):
+//   32:  3.2 + steps * (0.1 + 0.19 n), n >= 1, steps of 32 k:
+//        256x512x1536 17.3 -> 17.1, 1024x768x768 17.8 -> 19.3, 1024x2048x768 40 -> 42
+//   64:  4 + ceil(n) * (2.6 + 0.65 * blocks of 64 k):
+//        256x768x768 12.7 -> 14.4, 1024x2048x768 25.5 -> 24.8, 1024x4096x768 45.9 -> 45.6
+//   128: 5 + ceil(n) * (1.5 + 1.42 * steps), n >= 1.5:
+//        256x32000x288 36 -> 34, 1024x32000x768 277 -> 290
+//   split K: + 3 and the partials' traffic at 3.5 TB/s.
+// Without 16-byte rows the 32 tiles' loads cost 1.5x per step, the others' 1.2x
+// (501x517x1003: 24.8 against 16.9 µs with three splits).  The bf16 tiles keep
+// their partial sums at most as long as the fp32 tiles' would be (the 64
+// tile sums four of its own), so no result is summed in fewer pieces than before.
+struct GemmChoice { int tile, splits, k_per_split; float us, us32; };    // us32: the 32 tiles' estimate
+GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, bool vec, size_t ws_floats, int ek) {
+    const SplitPlan p = split_plan(op, M, N, K, ws_floats, ek);
+    const double mn = (double)M * N, cus = 256.0;
+    auto blocks = [&](int T) { return (double)((N + T - 1) / T) * ((M + T - 1) / T); };
+    auto reduce = [&](int s) { return s > 1 ? 3.0 + (s + 1) * mn * 4.0 / 3.5e6 : 0.0; };
+    auto steps = [&](int k, int per) { return (double)((k + per - 1) / per); };
+    const double us32 = 3.2 + reduce(p.splits) +
+                        (vec ? 1.0 : 1.5) * steps(p.k_per_split, BK) * (0.1 + 0.19 * std::max(1.0, blocks(32) * p.splits / cus));
+    GemmChoice best = {32, p.splits, p.k_per_split, (float)us32, (float)us32};
+    if (lda >= kMaxSplitLd || ldb >= kMaxSplitLd || (ek != GEMM_EPI_NONE && !vec)) return best;
+    // the large short-K weight gradients stay on the 128x96 fp32 tiles
+    // (32000x288x64: 22.4 us against 29.4)
+    if (op == 1 && vec && ek == GEMM_EPI_NONE && p.splits == 1 && mn >= (4L << 20) && K < 256) return best;
+    // long K and large NT outputs always leave the 32x32 tiles
+    const bool leave = K >= 4096 || (op == 2 && mn >= (4L << 20));
+    if (!leave && us32 < 7.0) return best;                       // below any of the others
+    if (leave) best.us = 1e30f;
+    const int max_s = ek != GEMM_EPI_NONE ? 1 : std::max(1, std::min(64, K / 128));
+    for (int s = 1; s <= max_s; s += 1 + s / 8) {
+        const double red = reduce(s);
+        if (s > 1 && ((size_t)s * M * N > std::min(ws_floats, kScratchFloats) || 7.0 + red > best.us)) break;
+        const int kps = ((K + s - 1) / s + BK - 1) / BK * BK, splits = (K + kps - 1) / kps;
+        for (int T = 64; T <= 128; T += 64) {
+            if (kps > (T == 64 ? 4 : 1) * p.k_per_split) continue;
+            const double n = blocks(T) * splits / cus;
+            if (T == 128 && n < 1.5) continue;
+            const double per = T == 64 ? 2.6 + 0.65 * steps(kps, 64) : 1.5 + 1.42 * steps(kps, BK);
+            const double us = (T == 64 ? 4.0 : 5.0) + (vec ? 1.0 : 1.2) * std::ceil(n) * per + red;
+            if (us < best.us) best = GemmChoice{T, splits, splits > 1 ? kps : K, (float)us, (float)us32};
+        }
+    }
+    if (best.tile == 32) best.us = (float)us32;
+    return best;
+}
+
 }  // namespace
 
 bool gemm_norm_fusable(int M, int N, int K, const float *A, long lda, const float *B, long ldb, int epi_kind,
                        const GemmNorm &nm) {
     if (nm.kind < GEMM_NORM_PLAIN || nm.kind > GEMM_NORM_EMBED || !nm.w || !nm.xn_out) return false;
     if (epi_kind != GEMM_EPI_ROPE && epi_kind != GEMM_EPI_SWIGLU) return false;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 4 || lda != K || ldb % 4 || ldb < K || gemm_big_tiles(2, M, N, K)) return false;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 4 || lda != K || ldb % 4 || ldb < K) return false;
     if (!A || !B || !al16(A) || !al16(B) || !al16(nm.w) || !al16(nm.xn_out)) return false;
+    // the fused norm runs on the 32x32 tiles only, and spares a launch (about 5 us)
+    const GemmChoice ch = gemm_choice(2, M, N, K, lda, ldb, true, 0, epi_kind);
+    if (ch.tile != 32 && ch.us + 5.0f < ch.us32) return false;
     if (nm.kind != GEMM_NORM_PLAIN && (!nm.x_out || !al16(nm.x_out))) return false;
     if (nm.kind == GEMM_NORM_SPLITS &&
         (nm.pk.splits < 1 || nm.pk.splits > kNormSplits || !nm.pk.parts || !al16(nm.pk.parts) || nm.pk.stride % 4 ||
@@ -989,49 +1326,38 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
     // extent that is a multiple of 4 (M for A^T, K for A; K for B^T, N for B)
     const bool vec = al16(A) && lda % 4 == 0 && (AT ? M : K) % 4 == 0 && al16(B) && ldb % 4 == 0 &&
                      (BT ? K : N) % 4 == 0;
-    // Kernel choice, measured on MI355X for the training shapes (graph-
-    // replayed launches): 32x32 tiles win everywhere except long K (>= 4096:
-    // 64x64 with K split over >= 512 blocks) and large NT outputs (>= 4M
-    // elements: 64x64).  Every small GEMM is bound by the latency of its K
-    // steps, so K is split when a 32x32 grid is small and K long: about
-    // eight K steps per split (K=768: 3 splits, K=864: 3, K=1536: 6).  With
-    // the panel kernel taking up to 9 K steps at once, eight per split ran
-    // the stories15M T=256 step in 0.769-0.771 ms against 0.778-0.783 with
-    // six (12.9 us less kernel time per step); nine and ten were no faster.
-    const bool big = gemm_big_tiles(op, M, N, K);
-    const int TM = big ? 64 : 32, TN = TM;
-    const int gx = (N + TN - 1) / TN, gy = (M + TM - 1) / TM;
-    const SplitPlan plan = split_plan(op, M, N, K, ws_floats, ek);
-    int splits = plan.splits;
-    g.k_per_split = plan.k_per_split;
+    // Kernel choice.  Small GEMMs are bound by the latency of their K steps
+    // and stay on 32x32 tiles (split_plan cuts K at about eight K steps per split:
+    // K=768: 3 splits, K=1536: 6; with the panel kernel taking up to 9 K
+    // steps at once, eight per split ran the stories15M T=256 step in
+    // 0.769-0.771 ms against 0.778-0.783 with six, and nine and ten were no
+    // faster); larger ones take the bf16-product tiles (gemm_choice).  The
+    // fused norm runs on the 32x32 tiles.
+    GemmChoice ch = gemm_choice(op, M, N, K, lda, ldb, vec, ws_floats, ek);
+    if (nk_kind && ch.tile != 32) ch = GemmChoice{32, 1, K, ch.us32, ch.us32};
+    const int T = ch.tile;
+    const int gx = (N + T - 1) / T, gy = (M + T - 1) / T;
+    const int splits = ch.splits;
+    g.k_per_split = ch.k_per_split;
     g.partial = splits > 1 ? ws : nullptr;
     g.epi = epi ? *epi : GemmEpi{};
     g.nrm = norm ? *norm : GemmNorm{};
-    if (gy > 65535) return set_error(PTMI_ERR_ARG, "gemm: M too large");
+    if ((M + 63) / 64 > 65535 || gy > 65535) return set_error(PTMI_ERR_ARG, "gemm: M too large");
     dim3 grid(gx, gy, splits);
     using KFn = void (*)(GemmArgs);
-    static const KFn kernels[2][2][3] = {
-        {{k_gemm<false, false, 32, 32, kRing32, false>, k_gemm<true, false, 32, 32, kRing32, false>,
-          k_gemm<false, true, 32, 32, kRing32, false>},
-         {k_gemm<false, false, 32, 32, kRing32, true>, k_gemm<true, false, 32, 32, kRing32, true>,
-          k_gemm<false, true, 32, 32, kRing32, true>}},
-        {{k_gemm<false, false, 64, 64, kRing64, false>, k_gemm<true, false, 64, 64, kRing64, false>,
-          k_gemm<false, true, 64, 64, kRing64, false>},
-         {k_gemm<false, false, 64, 64, kRing64, true>, k_gemm<true, false, 64, 64, kRing64, true>,
-          k_gemm<false, true, 64, 64, kRing64, true>}}};
-    KFn fn = kernels[big][vec][op];
+    static const KFn kernels[2][3] = {
+        {k_gemm<false, false, 32, 32, kRing32, false>, k_gemm<true, false, 32, 32, kRing32, false>,
+         k_gemm<false, true, 32, 32, kRing32, false>},
+        {k_gemm<false, false, 32, 32, kRing32, true>, k_gemm<true, false, 32, 32, kRing32, true>,
+         k_gemm<false, true, 32, 32, kRing32, true>}};
+    KFn fn = kernels[vec][op];
     if (ek != GEMM_EPI_NONE) {
-        static const KFn fused[2][2][2] = {
-            {{k_gemm<false, true, 32, 32, kRing32, false, GEMM_EPI_ROPE>, k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_ROPE>},
-             {k_gemm<false, true, 64, 64, kRing64, false, GEMM_EPI_ROPE>, k_gemm<false, true, 64, 64, kRing64, true, GEMM_EPI_ROPE>}},
-            {{k_gemm<false, true, 32, 32, kRing32, false, GEMM_EPI_SWIGLU>, k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_SWIGLU>},
-             {k_gemm<false, true, 64, 64, kRing64, false, GEMM_EPI_SWIGLU>, k_gemm<false, true, 64, 64, kRing64, true, GEMM_EPI_SWIGLU>}}};
-        static const KFn fused_nn[2][2] = {
-            {k_gemm<false, false, 32, 32, kRing32, false, GEMM_EPI_SWIGLU_BWD>,
-             k_gemm<false, false, 32, 32, kRing32, true, GEMM_EPI_SWIGLU_BWD>},
-            {k_gemm<false, false, 64, 64, kRing64, false, GEMM_EPI_SWIGLU_BWD>,
-             k_gemm<false, false, 64, 64, kRing64, true, GEMM_EPI_SWIGLU_BWD>}};
-        fn = ek == GEMM_EPI_SWIGLU_BWD ? fused_nn[big][vec] : fused[ek == GEMM_EPI_SWIGLU][big][vec];
+        static const KFn fused[2][2] = {
+            {k_gemm<false, true, 32, 32, kRing32, false, GEMM_EPI_ROPE>, k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_ROPE>},
+            {k_gemm<false, true, 32, 32, kRing32, false, GEMM_EPI_SWIGLU>, k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_SWIGLU>}};
+        static const KFn fused_nn[2] = {k_gemm<false, false, 32, 32, kRing32, false, GEMM_EPI_SWIGLU_BWD>,
+                                        k_gemm<false, false, 32, 32, kRing32, true, GEMM_EPI_SWIGLU_BWD>};
+        fn = ek == GEMM_EPI_SWIGLU_BWD ? fused_nn[vec] : fused[ek == GEMM_EPI_SWIGLU][vec];
     }
     if (nk_kind) {                                       // fusable: 32x32 float4 tiles, whole K
         static const KFn fused_norm[2][3] = {
@@ -1041,10 +1367,23 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
             {k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_SWIGLU, GEMM_NORM_PLAIN>,
              k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_SWIGLU, GEMM_NORM_SPLITS>,
              k_gemm<false, true, 32, 32, kRing32, true, GEMM_EPI_SWIGLU, GEMM_NORM_EMBED>}};
-        if (big || !vec || splits != 1) return set_error(PTMI_ERR_STATE, "gemm: fused norm without whole-K float4 tiles");
+        if (!vec || splits != 1) return set_error(PTMI_ERR_STATE, "gemm: fused norm without whole-K float4 tiles");
         fn = fused_norm[ek == GEMM_EPI_SWIGLU][nk_kind - 1];
     }
     int threads = 256;
+    if (T != 32) {
+#define PTMI_SPLIT_KERNELS(T_)                                                                                        \
+    {{k_gemm_split<false, true, T_, 1, 0>, k_gemm_split<true, true, T_, 1, 0>, k_gemm_split<false, false, T_, 1, 0>}, \
+     {k_gemm_split<false, true, T_, 4, 0>, k_gemm_split<true, true, T_, 4, 0>, k_gemm_split<false, false, T_, 4, 0>}}
+        static const KFn plain[2][2][3] = {PTMI_SPLIT_KERNELS(64), PTMI_SPLIT_KERNELS(128)};
+#undef PTMI_SPLIT_KERNELS
+        static const KFn fused[2][3] = {                 // by epilogue kind - 1
+            {k_gemm_split<false, false, 64, 4, GEMM_EPI_ROPE>, k_gemm_split<false, false, 64, 4, GEMM_EPI_SWIGLU>,
+             k_gemm_split<false, true, 64, 4, GEMM_EPI_SWIGLU_BWD>},
+            {k_gemm_split<false, false, 128, 4, GEMM_EPI_ROPE>, k_gemm_split<false, false, 128, 4, GEMM_EPI_SWIGLU>,
+             k_gemm_split<false, true, 128, 4, GEMM_EPI_SWIGLU_BWD>}};
+        fn = ek != GEMM_EPI_NONE ? fused[T == 128][ek - 1] : plain[T == 128][vec][op];
+    }
     // Per-layer 32x32 GEMMs with at most 9 K tiles per split: the panel
     // kernel, every K tile in flight at once.  PTMI_GEMM_PANEL is a bit mask
     // of the GEMMs that take it: 1 NT, 2 NN with the SwiGLU backward
@@ -1054,9 +1393,9 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
     // QKV dX) 82.0 -> 90.9, so those keep the ring.  Graph-mode step
     // 0.780-0.785 ms against 0.787-0.796 (mask 0) and 0.790-0.795 (mask 7).
     static const int use_panel = [] { const char *e = getenv("PTMI_GEMM_PANEL"); return e ? atoi(e) & 7 : 3; }();
-    const int nk_split = (plan.k_per_split + BK - 1) / BK;
+    const int nk_split = (ch.k_per_split + BK - 1) / BK;
     const int panel_bit = op == 2 ? 1 : ek == GEMM_EPI_SWIGLU_BWD ? 2 : 4;
-    if ((use_panel & panel_bit) && !big && vec && !nk_kind && op != 1 && nk_split <= 9) {
+    if ((use_panel & panel_bit) && T == 32 && vec && !nk_kind && op != 1 && nk_split <= 9) {
         using PFn = void (*)(GemmArgs);
         static const PFn panel[2][2][4] = {
             {{k_gemm_panel<false, 6, GEMM_EPI_NONE>, k_gemm_panel<false, 6, GEMM_EPI_ROPE>,
@@ -1069,18 +1408,12 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
         const PFn pf = panel[op == 0][nk_split > 6][ei];
         if (pf) fn = pf;
     }
-    // The large whole-K GEMMs without a fused epilogue (the classifier's
-    // forward and weight gradient) take the direct-to-LDS tiles.
-    if (vec && ek == GEMM_EPI_NONE && splits == 1 && (long)M * N >= (4L << 20)) {
-        if (op == 2 && M >= 192) {
-            grid = dim3((unsigned)((N + 127) / 128), (unsigned)((M + 255) / 256), 1);
-            fn = k_gemm_dl32<256, 128, 4, 2>;
-            threads = 512;
-        } else if (op == 1) {
-            grid = dim3((unsigned)((N + 95) / 96), (unsigned)((M + 127) / 128), 1);
-            fn = k_gemm_dl<true, true, 128, 96, 4, 2>;
-            threads = 512;
-        }
+    // The large short-K weight gradients (the classifier's at T <= 256) take
+    // the direct-to-LDS tiles.
+    if (T == 32 && vec && ek == GEMM_EPI_NONE && splits == 1 && op == 1 && (long)M * N >= (4L << 20)) {
+        grid = dim3((unsigned)((N + 95) / 96), (unsigned)((M + 127) / 128), 1);
+        fn = k_gemm_dl<true, true, 128, 96, 4, 2>;
+        threads = 512;
     }
     hipLaunchKernelGGL(fn, grid, dim3(threads), 0, s, g);
     PTMI_HIP(hipGetLastError());
@@ -1174,7 +1507,7 @@ size_t gemm_dev_ws_floats(int M, int N) {
 // process ends).  In host code `scratch` names a host-side stand-in, not
 // device memory: the device address comes from hipGetSymbolAddress, once
 // per device at ptmi_init, and only that address is handed to kernels.
-constexpr size_t kNoAllocScratchFloats = (size_t)4 << 20;
+constexpr size_t kNoAllocScratchFloats = kScratchFloats;
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) float scratch[kNoAllocScratchFloats];
 static float *g_scratch_dev[kMaxDevices] = {};

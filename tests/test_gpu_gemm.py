@@ -192,9 +192,8 @@ def test_gemm_dev_large_grids(op, M, N, K):
         a.free()
 
 
-# The direct-to-LDS tiles (NT with M >= 192 on 256x128 tiles, TN on 64x96;
-# outputs of 4M elements and more, whole K, no fused epilogue):
-# integer-exact at the classifier shapes of config 5, with and without
+# The largest outputs (4M elements and more: NT on the bf16-product tiles, TN
+# with K < 256 on the direct-to-LDS fp32 tiles): integer-exact at the classifier shapes of config 5, with and without
 # accumulate, and on ragged M, N and K.
 @pytest.mark.parametrize("op,M,N,K,acc", [(2, 256, 32000, 288, 0), (2, 256, 32000, 288, 1), (2, 193, 21845, 36, 1),
                                           (1, 32000, 288, 255, 0), (1, 32000, 288, 255, 1), (1, 16388, 260, 7, 0)])
@@ -238,6 +237,75 @@ def test_gemm_dev_panel_nt_exact(M, N, K, acc):
     assert np.array_equal(got, ref.astype(np.float32))
     for a in (dA, dB, dC):
         a.free()
+
+
+# The bf16-product tiles (middle and large GEMMs: 64x64 with K dealt to four
+# waves, 128x128 for many tiles): every op, whole and ragged M, N and K, K ranges
+# that leave a wave without work, split K, rows without 16-byte alignment,
+# padded leading dimensions, accumulate.
+SPLIT_TILES = [(0, 1024, 768, 2048, 0, 0), (1, 770, 2050, 1000, 1, 2), (2, 1024, 2048, 768, 1, 0), (2, 333, 8001, 701, 0, 0),
+               (0, 501, 517, 1003, 1, 0), (1, 1003, 517, 501, 0, 1), (0, 65, 4100, 4097, 0, 3), (2, 200, 32000, 300, 1, 0),
+               (1, 33000, 130, 300, 0, 0), (2, 257, 21847, 37, 0, 0), (0, 700, 12000, 260, 0, 4), (2, 64, 65600, 20, 0, 0)]
+
+
+def split_tile_call(op, A, B, C0, M, N, K, acc, pad):
+    """C (+)= op(A).op(B) of dense A [M,K], B [K,N] through ptmi_gemm_dev,
+    operands stored as `op` wants them with `pad` NaN columns after each row."""
+    def stored(x):
+        return np.ascontiguousarray(np.pad(x, ((0, 0), (0, pad)), constant_values=np.nan), np.float32)
+    a, b, c = stored(A.T if op == 1 else A), stored(B.T if op == 2 else B), stored(C0)
+    dA, dB, dC = DeviceArray.from_host(a), DeviceArray.from_host(b), DeviceArray.from_host(c)
+    L = pa.load_ptmi()
+    assert L.ptmi_gemm_dev(op, dA.ptr, a.shape[1], dB.ptr, b.shape[1], dC.ptr, N + pad, M, N, K, acc, None) == 0
+    assert L.ptmi_sync() == 0
+    got = dC.download().reshape(M, N + pad)[:, :N]
+    for d in (dA, dB, dC):
+        d.free()
+    return got
+
+
+@pytest.mark.parametrize("op,M,N,K,acc,pad", SPLIT_TILES)
+def test_gemm_dev_split_tiles_exact(op, M, N, K, acc, pad):
+    A, B = ints((M, K), 41), ints((K, N), 42)
+    C0 = ints((M, N), 43) if acc else np.full((M, N), np.nan, np.float32)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    got = split_tile_call(op, A, B, C0, M, N, K, acc, pad)
+    assert np.array_equal(got, (ref + C0 if acc else ref).astype(np.float32))
+
+
+@pytest.mark.parametrize("op,M,N,K,acc,pad", SPLIT_TILES)
+def test_gemm_dev_split_tiles_keep_all_bits(op, M, N, K, acc, pad):
+    """One operand random in all 24 bits over 60 binades, the other with one
+    power of two per sum: every result is a single product and exact."""
+    rng = np.random.default_rng(K)
+    full = lambda shape: (rng.uniform(1, 2, shape) * 2.0 ** rng.integers(-30, 30, shape) * rng.choice((-1, 1), shape)).astype(np.float32)
+    C0 = np.zeros((M, N), np.float32)
+    A, B = full((M, K)), np.zeros((K, N), np.float32)
+    at, sc = rng.integers(0, K, N), (2.0 ** rng.integers(-20, 20, N)).astype(np.float32)
+    B[at, np.arange(N)] = sc
+    assert np.array_equal(split_tile_call(op, A, B, C0, M, N, K, 0, pad), A[:, at] * sc)
+    A, B = np.zeros((M, K), np.float32), full((K, N))
+    at, sc = rng.integers(0, K, M), (2.0 ** rng.integers(-20, 20, M)).astype(np.float32)
+    A[np.arange(M), at] = sc
+    assert np.array_equal(split_tile_call(op, A, B, C0, M, N, K, 0, pad), B[at] * sc[:, None])
+
+
+@pytest.mark.parametrize("op,M,N,K,acc,pad", [SPLIT_TILES[i] for i in (0, 3, 4, 7, 8)])
+def test_gemm_dev_split_tiles_non_finite(op, M, N, K, acc, pad):
+    """Infinities, NaNs and numbers next to the largest give what a product
+    and sum in fp32 gives, and leave the other rows and columns alone."""
+    rng = np.random.default_rng(M)
+    A, B = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(0.5, 1, (K, N)).astype(np.float32)
+    A[3, 5], A[17, K - 1], A[M - 1, 0] = np.inf, -np.inf, np.nan
+    A[9, 2], A[10, 2], A[10, 3] = np.finfo(np.float32).max, np.inf, -np.inf
+    B[2, 7] = 0.25
+    C0 = np.zeros((M, N), np.float32)
+    got = split_tile_call(op, A, B, C0, M, N, K, 0, pad)
+    assert np.all(np.isposinf(got[3])) and np.all(np.isneginf(got[17]))
+    assert np.all(np.isnan(got[M - 1])) and np.all(np.isnan(got[10]))
+    clean = np.setdiff1d(np.arange(M), (3, 10, 17, M - 1))
+    a, b = A[clean].astype(np.float64), B.astype(np.float64)
+    assert bound_ok(got[clean], a @ b, np.abs(a) @ np.abs(b), K)
 
 
 def test_gemm_errors():
