@@ -62,3 +62,27 @@ def test_different_blob_at_a_held_address_is_refused():
     assert L.ptmi_unregister_weights(P(blob)) == 0
     assert L.ptmi_unregister_weights(P(blob)) == 0
     assert L.ptmi_unregister_weights(P(blob)) == ERR_ARG
+
+
+# w1 and w3 pass through a 4 Mi-float staging buffer: less than one fill,
+# a little more than one, and several with a ragged last one.
+@pytest.mark.parametrize("cfg", [(8, 4, 1, 2, 2, 16, 4), (64, 2048, 33, 4, 4, 16, 4), (260, 2002, 17, 5, 5, 64, 4)])
+def test_weights_round_trip(cfg):
+    blob = pa.synth_model(cfg, 8)
+    if cfg[1] % 4:                                   # not a model shape: through the matvec's view of the registration
+        L = pa.load_ptmi()
+        D, H, n_l = cfg[:3]
+        assert L.ptmi_register_weights(P(blob), blob.nbytes) == 0
+        w = blob[28:].view(np.float32)
+        w1 = cfg[5] * D + 4 * n_l * D * D + 2 * n_l * D
+        x = np.zeros(D, np.float32)
+        x[D - 1] = 1.0
+        for block, off in (("w1", w1), ("w3", w1 + 2 * n_l * H * D)):
+            for layer in (0, 1, n_l // 2, n_l - 1):
+                W = w[off + layer * H * D:off + (layer + 1) * H * D].reshape(H, D)
+                assert np.array_equal(pa.matvec(W, x), W[:, D - 1]), (block, layer)
+        assert L.ptmi_unregister_weights(P(blob)) == 0
+        return
+    m = pa.Model(blob)
+    assert np.array_equal(m.read_weights(), blob)
+    m.close()
