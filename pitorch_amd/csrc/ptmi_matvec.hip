@@ -321,51 +321,120 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecParams p) {
     if (active) run_epilogue<EPI>(p, ybuf[wave], row0, nrows, lane, pos, res);
 }
 
-// Long rows (n > 64*9*4): one wave per row pair, x read through the cache
-// in 64-chunk strides.  Used by the drop-in path for transposed weights
-// (e.g. W_cls^T, in_dim = vocab) — not by the decode step.
-__global__ __launch_bounds__(256) void k_matvec_long(MatvecParams p) {
-    __shared__ float ybuf[kWaves][kMaxRowsPerWave];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int n4 = p.n >> 2;
-    const long wave_id = (long)blockIdx.x * kWaves + wave;
-    const long row0l = wave_id * p.rows_per_wave;
-    const bool active = row0l < p.rows;
-    const int row0 = active ? (int)row0l : 0;
-    const int nrows = active ? min(p.rows_per_wave, p.rows - row0) : 0;
-    const float4 *x4 = reinterpret_cast<const float4 *>(p.x);
-    for (int r = 0; r < nrows; r += 2) {
-        const bool vb = r + 1 < nrows;
-        const float4 *wa = reinterpret_cast<const float4 *>(p.W + (long)(row0 + r) * p.ld);
-        const float4 *wb = reinterpret_cast<const float4 *>(p.W + (long)(row0 + (vb ? r + 1 : r)) * p.ld);
-        float a = 0.0f, b = 0.0f;
-        for (int c = lane; c < n4; c += 64) {
-            const float4 xv = x4[c];
-            a = dot4(wa[c], xv, a);
-            b = dot4(wb[c], xv, b);
-        }
-        a = group_sum<64>(a);
-        b = group_sum<64>(b);
-        if (lane == 0) {
-            ybuf[wave][r] = a;
-            if (vb) ybuf[wave][r + 1] = b;
-        }
-    }
-    __syncthreads();
-    if (active) run_epilogue<EPI_STORE>(p, ybuf[wave], row0, nrows, lane, 0, 0.0f);
+// Plain matvecs outside the register-resident kernel's range: rows longer than
+// 64*9*4 floats, and rows whose start or length is no multiple of 16 bytes.
+// 16-byte loads need 4-byte alignment only, so both stream whole float4s from
+// wherever the row starts; the last n % 4 elements follow one per lane.  As
+// above, chunks past the row are loaded from its last chunk and dropped by a
+// select, so that all loads of a pass are in flight together.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef floatx4 __attribute__((aligned(4))) floatx4_any;
+
+__device__ __forceinline__ floatx4 load4_any(const float *p) { return *reinterpret_cast<const floatx4_any *>(p); }
+__device__ __forceinline__ floatx4 stream4_any(const float *p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const floatx4_any *>(p));
+}
+__device__ __forceinline__ floatx4 keep4(bool keep, floatx4 v) {
+    return floatx4{keep ? v.x : 0.0f, keep ? v.y : 0.0f, keep ? v.z : 0.0f, keep ? v.w : 0.0f};
+}
+__device__ __forceinline__ float fma4(floatx4 w, floatx4 x, float acc) {
+    acc = fmaf(w.x, x.x, acc);
+    acc = fmaf(w.y, x.y, acc);
+    acc = fmaf(w.z, x.z, acc);
+    return fmaf(w.w, x.w, acc);
+}
+__device__ __forceinline__ void store_row(const MatvecParams &p, long r, float v) {
+    p.y[r] = p.epi == EPI_RESIDUAL ? p.y[r] + v : v;
 }
 
-// Any alignment / any n: one wave per row, scalar loads.
-__global__ __launch_bounds__(256) void k_matvec_scalar(MatvecParams p) {
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (row >= p.rows) return;
-    const float *w = p.W + row * p.ld;
-    float a = 0.0f;
-    for (int j = lane; j < p.n; j += 64) a = fmaf(w[j], p.x[j], a);
-    a = group_sum<64>(a);
-    if (lane == 0) p.y[row] = (p.epi == EPI_RESIDUAL) ? p.y[row] + a : a;
+// Long rows: a block of W waves takes RB rows, its waves interleaved passes of 4
+// float4 per lane and row, so a few hundred rows already fill the chip (one
+// wave per row pair kept 384 waves with one load pair each in flight on 768
+// rows).  Measured: 768x32000 (the transposed classifier) 66 -> 18 us (5.4 TB/s;
+// a lone launch reaches 6.0), 288x32000 9.7, 2048x4096 7.0, 4000x8003 21.7.
+template <int W, int RB>
+__global__ __launch_bounds__(64 * W) void k_matvec_long(MatvecParams p) {
+    constexpr int U = 4;
+    __shared__ float part[W][RB];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n4 = p.n >> 2;
+    const long r0 = (long)blockIdx.x * RB;
+    const float *w[RB];
+    float acc[RB];
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+        w[r] = p.W + min(r0 + r, (long)p.rows - 1) * p.ld;
+        acc[r] = 0.0f;
+    }
+    for (int c0 = wave * 64 * U + lane; c0 - lane < n4; c0 += W * 64 * U) {
+        floatx4 wv[RB][U], xv[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int r = 0; r < RB; r++) wv[r][u] = stream4_any(w[r] + 4L * min(c0 + 64 * u, n4 - 1));
+#pragma unroll
+        for (int u = 0; u < U; u++) xv[u] = load4_any(p.x + 4L * min(c0 + 64 * u, n4 - 1));
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool in = c0 + 64 * u < n4;
+            const floatx4 x = keep4(in, xv[u]);
+#pragma unroll
+            for (int r = 0; r < RB; r++) acc[r] = fma4(keep4(in, wv[r][u]), x, acc[r]);
+        }
+    }
+    const int j = 4 * n4 + lane;
+    if (wave == W - 1 && j < p.n) {
+        const float x = p.x[j];
+#pragma unroll
+        for (int r = 0; r < RB; r++) acc[r] = fmaf(w[r][j], x, acc[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+        const float s = group_sum<64>(acc[r]);
+        if (lane == 0) part[wave][r] = s;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < RB && r0 + threadIdx.x < p.rows) {
+        float s = part[0][threadIdx.x];
+#pragma unroll
+        for (int k = 1; k < W; k++) s += part[k][threadIdx.x];
+        store_row(p, r0 + threadIdx.x, s);
+    }
+}
+
+// Rows of at most 64*9*4 floats at any alignment: RW rows per wave, IT float4 of
+// each per lane (IT = ceil(n/4 / 64), 0 where n < 4), everything loaded before
+// any of it is used.  5003x1027 with 4-byte loads one after another: 7.1 us, now 5.1
+// (4.0 TB/s); 30001x301 7.8, 20001x101 4.1.
+template <int IT, int RW>
+__global__ __launch_bounds__(256) void k_matvec_any(MatvecParams p) {
+    const int lane = threadIdx.x & 63, n4 = p.n >> 2, tail = p.n & 3;
+    const long r0 = ((long)blockIdx.x * kWaves + (threadIdx.x >> 6)) * RW;
+    if (r0 >= p.rows) return;
+    floatx4 wv[RW][IT ? IT : 1], xv[IT ? IT : 1];
+    float wt[RW];
+    const int jt = min(4 * n4 + (lane & 3), p.n - 1);            // inside the row for every lane
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        const float *w = p.W + min(r0 + r, (long)p.rows - 1) * p.ld;
+#pragma unroll
+        for (int i = 0; i < IT; i++) wv[r][i] = stream4_any(w + 4 * min(i * 64 + lane, n4 - 1));
+        wt[r] = w[jt];
+    }
+#pragma unroll
+    for (int i = 0; i < IT; i++) xv[i] = load4_any(p.x + 4 * min(i * 64 + lane, n4 - 1));
+    const float xt = p.x[jt];
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        float a = lane < tail ? wt[r] * xt : 0.0f;
+#pragma unroll
+        for (int i = 0; i < IT; i++) {
+            const bool in = i * 64 + lane < n4;
+            a = fma4(keep4(in, wv[r][i]), keep4(in, xv[i]), a);
+        }
+        a = group_sum<64>(a);
+        if (lane == 0 && r0 + r < p.rows) store_row(p, r0 + r, a);
+    }
 }
 
 using KernelFn = void (*)(MatvecParams);
@@ -426,6 +495,22 @@ KernelFn pick_xr_np(int it) {
 template <int LPR>
 KernelFn pick_xr(int it, int np) {
     return np == 2 ? pick_xr_np<LPR, 2>(it) : pick_xr_np<LPR, 1>(it);
+}
+
+template <int RW>
+KernelFn pick_any(int it) {
+    switch (it) {
+    case 0: return k_matvec_any<0, RW>;
+    case 1: return k_matvec_any<1, RW>;
+    case 2: return k_matvec_any<2, RW>;
+    case 3: return k_matvec_any<3, RW>;
+    case 4: return k_matvec_any<4, RW>;
+    case 5: return k_matvec_any<5, RW>;
+    case 6: return k_matvec_any<6, RW>;
+    case 7: return k_matvec_any<7, RW>;
+    case 8: return k_matvec_any<8, RW>;
+    default: return k_matvec_any<9, RW>;
+    }
 }
 
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -580,7 +665,6 @@ int launch_matvec(MatvecParams p, hipStream_t s, hipEvent_t e0, hipEvent_t e1, b
         return set_error(PTMI_ERR_ARG, "matvec: SwiGLU needs an even row count");
 
     KernelFn fn = nullptr;
-    int rpp = 1;
     MatvecGeom geo;
     if (x_reread && (p.pro != PRO_NONE || p.epi != EPI_STORE || p.pf.blocks))
         return set_error(PTMI_ERR_ARG, "matvec: the x re-read variant is a plain y = Wx");
@@ -611,34 +695,35 @@ int launch_matvec(MatvecParams p, hipStream_t s, hipEvent_t e0, hipEvent_t e1, b
         launch_k(fn, dim3((unsigned)(compute_blocks + p.pf.blocks)), dim3(geo.wpb * 64), 0, s, e0, e1, p);
         PTMI_HIP(hipGetLastError());
         return PTMI_OK;
-    } else if (x_reread) {
+    }
+    if (x_reread)
         return set_error(PTMI_ERR_ARG, "matvec: the x re-read variant needs 16-byte rows of n <= %d", 64 * 9 * 4);
-    } else if (vec_ok) {
+    if (vec_ok) {
         if (p.pf.blocks) return set_error(PTMI_ERR_ARG, "matvec: prefetch needs the register-resident kernel");
         if (p.pro != PRO_NONE || p.epi != EPI_STORE)
             return set_error(PTMI_ERR_ARG, "matvec: fused variants need n <= %d", 64 * 9 * 4);
-        fn = k_matvec_long;
-        rpp = 1;
-    } else {
-        if (fused) return set_error(PTMI_ERR_ARG, "matvec: fused variants need 16-byte aligned rows, n%%4==0");
-        p.rows_per_wave = 1;
-        const int blocks = (p.rows + kWaves - 1) / kWaves;
-        launch_k(k_matvec_scalar, dim3(blocks), dim3(kWaves * 64), 0, s, e0, e1, p);
-        PTMI_HIP(hipGetLastError());
-        return PTMI_OK;
+    } else if (fused) {
+        return set_error(PTMI_ERR_ARG, "matvec: fused variants need 16-byte aligned rows, n%%4==0");
     }
-    // rows per wave: a multiple of 2*rpp (row pairs for the fused epilogues),
-    // at most 64, chosen for ~2048 waves in flight.
-    const int step = 2 * rpp;
-    const long target_waves = 2048;
-    long rpw = (p.rows + target_waves - 1) / target_waves;
-    rpw = ((rpw + step - 1) / step) * step;
-    rpw = std::max<long>(rpw, step);
-    rpw = std::min<long>(rpw, kMaxRowsPerWave);
-    p.rows_per_wave = (int)rpw;
-    const long waves = (p.rows + rpw - 1) / rpw;
-    const long blocks = (waves + kWaves - 1) / kWaves;
-    launch_k(fn, dim3((unsigned)blocks), dim3(kWaves * 64), 0, s, e0, e1, p);
+    if (p.n > 64 * 9 * 4) {
+        // Two rows per block share their x, unless one row each leaves less
+        // on the fullest of the 256 CUs (768 rows: 3 against 4 rows, 18.0 against
+        // 19.0 us; 288 rows: 2 and 2, 11.3 against 9.7).  Eight waves where a
+        // row gives each of them a whole pass.
+        const bool two = (((long)p.rows + 1) / 2 + 255) / 256 * 2 <= ((long)p.rows + 255) / 256;
+        const bool eight = p.n >= 8192;
+        fn = eight ? (two ? k_matvec_long<8, 2> : k_matvec_long<8, 1>) : (two ? k_matvec_long<4, 2> : k_matvec_long<4, 1>);
+        const long blocks = two ? ((long)p.rows + 1) / 2 : p.rows;
+        launch_k(fn, dim3((unsigned)blocks), dim3(eight ? 512 : 256), 0, s, e0, e1, p);
+    } else {
+        // one row per wave up to kBigWaves of them, then two and (short
+        // rows, whose loads leave registers for it) four
+        const int it = (p.n / 4 + 63) / 64;
+        const int rw = p.rows <= kBigWaves ? 1 : p.rows <= 2 * kBigWaves || it > 4 ? 2 : 4;
+        fn = rw == 1 ? pick_any<1>(it) : rw == 2 ? pick_any<2>(it) : pick_any<4>(it);
+        const long per = (long)kWaves * rw, blocks = (p.rows + per - 1) / per;
+        launch_k(fn, dim3((unsigned)blocks), dim3(kWaves * 64), 0, s, e0, e1, p);
+    }
     PTMI_HIP(hipGetLastError());
     return PTMI_OK;
 }

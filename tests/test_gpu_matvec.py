@@ -66,6 +66,37 @@ def test_long_rows_and_unaligned_views():
     check_close(pa.matvec(Wv, x), oracle_mv(np.ascontiguousarray(Wv), x), Wv, x)
 
 
+# Rows outside the register-resident kernel's range: lengths around each
+# kernel's passes (4 floats a lane, 256 a wave, 2304, 4096, 8192), row counts
+# around the rows per wave and block, odd row strides and starts.  The
+# padding between rows and around them is NaN.
+@pytest.mark.parametrize("d,n,pad,start", [(1, 1, 0, 0), (7, 3, 2, 1), (5, 5, 0, 3), (9, 255, 1, 2), (8193, 257, 0, 1),
+                                           (20001, 101, 0, 0), (16385, 1029, 3, 1), (301, 2303, 0, 1), (6, 2304, 1, 0),
+                                           (1, 2305, 0, 0), (511, 2308, 4, 0), (513, 4099, 1, 3), (257, 8191, 0, 0),
+                                           (3, 8193, 0, 2), (768, 16387, 5, 1), (288, 32000, 0, 0)])
+def test_any_row_length_stride_and_start(d, n, pad, start):
+    from pitorch_amd._hip import DeviceArray
+    L = pa.load_ptmi()
+    rng = np.random.default_rng(n)
+    ld = n + pad
+    buf = np.full(start + d * ld + 8, np.nan, np.float32)
+    rows = buf[start:start + d * ld].reshape(d, ld)
+    rows[:, :n] = rng.uniform(-1, 1, (d, n))
+    W, x = np.ascontiguousarray(rows[:, :n]), rng.uniform(-1, 1, n).astype(np.float32)
+    xb = np.full(start + n + 8, np.nan, np.float32)
+    xb[start:start + n] = x
+    dW, dx, dy = DeviceArray.from_host(buf), DeviceArray.from_host(xb), DeviceArray.from_host(np.full(d + 1, -7, np.float32))
+    assert L.ptmi_matvec_dev(dW.ptr + 4 * start, ld, dx.ptr + 4 * start, dy.ptr, d, n, None) == 0
+    assert L.ptmi_sync() == 0
+    y = dy.download()
+    assert y[d] == -7
+    exact = W.astype(np.float64) @ x.astype(np.float64)
+    gamma = n * 2.0 ** -24 / (1 - n * 2.0 ** -24)
+    assert (np.abs(y[:d] - exact) <= gamma * (np.abs(W) @ np.abs(x)) + 1e-30).all()
+    for a in (dW, dx, dy):
+        a.free()
+
+
 def test_bad_arguments_are_errors():
     L = pa.load_ptmi()
     W = np.ones((4, 4), np.float32)
