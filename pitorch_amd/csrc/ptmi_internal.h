@@ -424,6 +424,34 @@ int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host
 // Entries [i0, i1) of a prepared table, whose tiles number `tiles`.
 int launch_gemm_tn_group(const void *dev_desc, int i0, int i1, int tiles, int vec, hipStream_t s);
 
+// Causal attention of all heads over `rows` positions on the matrix cores
+// (head_dim a multiple of 4, at most 128; row strides and head_dim multiples
+// of 4 floats, rows 16-byte aligned).
+struct AttnFwdArgs {
+    const float *q; long ldq;          // row r, head h: q + r*ldq + h*head_dim; its position is pos0 + r
+    const float *k, *v; long ldkv;     // positions 0 .. pos0 + rows - 1
+    float *out; long ldo;
+    float *row_max, *row_inv;          // [heads][stat_ld] kept for the backward: row maximum, 1/sum (null: not kept)
+    long stat_ld;
+    int rows, pos0, head_dim;
+    float scale;
+};
+int launch_attn_fwd(const AttnFwdArgs &a, int heads, hipStream_t s);
+// The gradients of q, k and v (rope_backward applied to dq and dk) for rows
+// [q | k | v] of `dim` columns each.  delta: [heads][stat_ld] scratch.  The
+// statistics rows hold at least `rows` rounded up to 16 floats.
+struct AttnBwdArgs {
+    const float *qkv; long ldqkv;
+    const float *out, *d_out;          // [rows][dim]
+    const float *row_max, *row_inv;
+    float *delta;
+    long stat_ld;
+    float *d_qkv;                      // row stride ldqkv
+    int rows, dim, head_dim;
+    float scale;
+};
+int launch_attn_bwd(const AttnBwdArgs &a, int heads, hipStream_t s);
+
 // ── library state ───────────────────────────────────────────────────────
 struct Config {
     int dim, hidden, n_layers, n_heads, n_kv_heads, vocab, seq_len;

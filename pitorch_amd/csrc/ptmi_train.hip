@@ -34,7 +34,10 @@ struct TrainState {
     // written once per step: d_res and d_xb by version (one per RMSNorm
     // backward, 2L+1, plus d_res's zero start), d_h13, sh and d_qkv per
     // layer, the RMSNorm inverse norms per norm.
-    float *d_res, *d_xb, *d_sh, *d_h13, *shb, *d_aout, *d_q, *d_k, *d_v, *d_qkv, *ds, *row_inv, *row_loss, *loss;
+    float *d_res, *d_xb, *d_sh, *d_h13, *shb, *d_aout, *d_qkv, *ds, *row_inv, *row_loss, *loss;
+    // Tiled attention: row maxima, then 1/sums, [layer][head][T rounded up to
+    // 16] each, and the backward's per-row dot products.
+    float *stat, *delta;
     // Descriptor tables of the two grouped launches (device; built per T).
     void *dw_desc;
     float *nd_desc;
@@ -150,111 +153,6 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(float *in, const float *w,
     ss = block_sum<4>(ss, red);
     const float inv = 1.0f / d_sqrtf(ss / D + 1e-5f);
     for (int i = threadIdx.x; i < D; i += 256) out[r + i] = x[i] * inv * w[i];
-}
-
-// Attention blocks: 256 threads; G lanes (G*4 >= head_dim) hold one
-// position's head row as float4, so a wave covers 64/G positions per load
-// and the block 256/G.
-constexpr int kAttnThreads = 256;
-
-// Per-position dot products s[t2] = a . B[t2] (B rows at b + t2*ld) for t2
-// in [0, n), G lanes per row; lane sub's float4 of `a` is a4.
-template <int G>
-__device__ __forceinline__ void row_dots(const float *b, long ld, float4 a4, int hd4, int n, float *out, float mul) {
-    constexpr int S = kAttnThreads / G;
-    const int slot = threadIdx.x / G, sub = threadIdx.x % G;
-    const bool has = sub < hd4;
-    for (int base = 0; base < n; base += 4 * S) {
-        float4 r[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int t2 = min(base + u * S + slot, n - 1);
-            r[u] = has ? reinterpret_cast<const float4 *>(b + (long)t2 * ld)[sub] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            float v = has ? dot4(a4, r[u]) : 0.0f;
-            v = group_sum<G>(v);
-            const int t2 = base + u * S + slot;
-            if (sub == 0 && t2 < n) out[t2] = v * mul;
-        }
-    }
-}
-
-// o[i] = sum_{t2 < n} w[t2] B[t2][i] for i < hd (B rows at b + t2*ld); the
-// 256/G slots take interleaved positions and their partial sums meet in
-// LDS `part` (at least (256/G)*hd floats).  Thread i < hd returns o[i].
-constexpr int kAttnPart = 1024;   // (256/G) * hd <= 1024 for hd <= 4*G
-template <int G>
-__device__ __forceinline__ float weighted_rows(const float *b, long ld, const float *w, int hd4, int n, float *part) {
-    constexpr int S = kAttnThreads / G;
-    const int slot = threadIdx.x / G, sub = threadIdx.x % G;
-    const bool has = sub < hd4;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int base = 0; base < n; base += 4 * S) {
-        float4 r[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int t2 = min(base + u * S + slot, n - 1);
-            r[u] = has ? reinterpret_cast<const float4 *>(b + (long)t2 * ld)[sub] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int t2 = base + u * S + slot;
-            const float e = t2 < n ? w[t2] : 0.0f;
-            acc.x += e * r[u].x;
-            acc.y += e * r[u].y;
-            acc.z += e * r[u].z;
-            acc.w += e * r[u].w;
-        }
-    }
-    const int hd = 4 * hd4;
-    __syncthreads();                      // earlier readers of part are done
-    if (has) reinterpret_cast<float4 *>(part + slot * hd)[sub] = acc;
-    __syncthreads();
-    float o = 0.0f;
-    if ((int)threadIdx.x < hd) {
-        o = part[threadIdx.x];
-        for (int k = 1; k < S; k++) o += part[k * hd + threadIdx.x];
-    }
-    return o;
-}
-
-// Causal attention for one (position t, head h): pt_train.c:224-255.
-// Dynamic LDS: sc[T].
-template <int G>
-__global__ __launch_bounds__(kAttnThreads) void k_attn_fwd(const float *qkv, float *att, float *att_out, int T, int D,
-                                                           int QS, int KV, int hd, int kv_mul, float scale) {
-    extern __shared__ float sc[];
-    __shared__ float part[kAttnPart];
-    __shared__ float red[4];
-    const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, hd4 = hd >> 2, sub = tid % G;
-    const int ko = D + (h / kv_mul) * hd, vo = D + KV + (h / kv_mul) * hd;
-    const float4 q4 = sub < hd4 ? reinterpret_cast<const float4 *>(qkv + (long)t * QS + h * hd)[sub]
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-    const int n = t + 1;
-    row_dots<G>(qkv + ko, QS, q4, hd4, n, sc, scale);
-    __syncthreads();
-    float mx = -INFINITY;
-    for (int t2 = tid; t2 < n; t2 += kAttnThreads) mx = fmaxf(mx, sc[t2]);
-    mx = block_max<4>(mx, red);
-    float sum = 0.0f;
-    for (int t2 = tid; t2 < n; t2 += kAttnThreads) {
-        const float e = d_expf(sc[t2] - mx);
-        sc[t2] = e;
-        sum += e;
-    }
-    sum = block_sum<4>(sum, red);
-    const float inv = 1.0f / sum;
-    float *arow = att + ((long)h * T + t) * T;
-    for (int t2 = tid; t2 < T; t2 += kAttnThreads) {
-        const float a = t2 < n ? sc[t2] * inv : 0.0f;
-        arow[t2] = a;
-        if (t2 < n) sc[t2] = a;
-    }
-    __syncthreads();
-    const float o = weighted_rows<G>(qkv + vo, QS, sc, hd4, n, part);
-    if (tid < hd) att_out[(long)t * D + h * hd + tid] = o;
 }
 
 // Cross-entropy row t < T-1 (pt_train.c:310-325) and, in place, its loss
@@ -592,68 +490,11 @@ __device__ __forceinline__ void rmsnorm_dw_block(const NormDw *nd, int cb, int R
     }
 }
 
-// Attention backward, row half (pt_train.c:780-811): for (t < R, head h):
-// d_att_s, the softmax backward dot, ds = d_pre*scale (kept for the column
-// half) and d_q[t] = sum_t2 ds[t2] k[t2].  Dynamic LDS: das[T].
-template <int G>
-__global__ __launch_bounds__(kAttnThreads) void k_attn_bwd_rows(const float *qkv, const float *att,
-                                                                const float *d_aout, float *ds, float *d_q, int T,
-                                                                int D, int QS, int KV, int hd, int kv_mul,
-                                                                float scale) {
-    extern __shared__ float das[];
-    __shared__ float part[kAttnPart];
-    __shared__ float red[4];
-    const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, hd4 = hd >> 2, sub = tid % G;
-    const float *arow = att + ((long)h * T + t) * T;
-    const int ko = D + (h / kv_mul) * hd, vo = D + KV + (h / kv_mul) * hd;
-    const float4 g4 = sub < hd4 ? reinterpret_cast<const float4 *>(d_aout + (long)t * D + h * hd)[sub]
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-    const int n = t + 1;
-    row_dots<G>(qkv + vo, QS, g4, hd4, n, das, 1.0f);
-    __syncthreads();
-    float dot = 0.0f;
-    for (int t2 = tid; t2 < n; t2 += kAttnThreads) dot += das[t2] * arow[t2];
-    dot = block_sum<4>(dot, red);
-    float *dsrow = ds + ((long)h * T + t) * T;
-    for (int t2 = tid; t2 < n; t2 += kAttnThreads) {
-        const float d = arow[t2] * (das[t2] - dot) * scale;
-        das[t2] = d;
-        dsrow[t2] = d;
-    }
-    __syncthreads();
-    const float o = weighted_rows<G>(qkv + ko, QS, das, hd4, n, part);
-    if (tid < hd) d_q[(long)t * D + h * hd + tid] = o;
-}
-
-// Attention backward, column half: for (t2 < R, head h):
-// d_v[t2] = sum_{t>=t2} att[t][t2] d_aout[t],  d_k[t2] = sum_{t>=t2} ds[t][t2] q[t].
-// Dynamic LDS: w[2*T].
-template <int G>
-__global__ __launch_bounds__(kAttnThreads) void k_attn_bwd_cols(const float *qkv, const float *att, const float *ds,
-                                                                const float *d_aout, float *d_k, float *d_v, int T,
-                                                                int R, int D, int QS, int KV, int hd, int kv_mul) {
-    extern __shared__ float sm[];
-    __shared__ float part[kAttnPart];
-    float *wa = sm, *wd = sm + T;
-    const int t2 = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, hd4 = hd >> 2;
-    const int kvo = (h / kv_mul) * hd, n = R - t2;
-    for (int k = tid; k < n; k += kAttnThreads) {
-        const long a = ((long)h * T + t2 + k) * T + t2;
-        wa[k] = att[a];
-        wd[k] = ds[a];
-    }
-    __syncthreads();
-    const float dv = weighted_rows<G>(d_aout + (long)t2 * D + h * hd, D, wa, hd4, n, part);
-    const float dk = weighted_rows<G>(qkv + (long)t2 * QS + h * hd, QS, wd, hd4, n, part);
-    if (tid < hd) {
-        d_v[(long)t2 * KV + kvo + tid] = dv;
-        d_k[(long)t2 * KV + kvo + tid] = dk;
-    }
-}
-
-// ── attention on the matrix cores ────────────────────────────────────────
-// The same three attention kernels for head_dim = 16*HQ (HQ <= 8), with
-// n_kv_heads == n_heads (training requires it), on v_mfma_f32_16x16x4_f32.
+// ── attention with whole score rows in LDS ───────────────────────────────
+// Three attention kernels for short sequences (lds_rows_attention; the
+// others take the tiled ones of ptmi_attention.hip), head_dim = 16*HQ
+// (HQ <= 8), n_kv_heads == n_heads (training requires it), on
+// v_mfma_f32_16x16x4_f32.
 // One block of kMW waves per (16-row tile, head).  Lane l supplies
 // A[l%16][l/16] and B[l/16][l%16]; result register r of lane l is
 // C[4*(l/16)+r][l%16].  A and B may share any order of the contraction
@@ -671,6 +512,16 @@ constexpr int kMW = 8, kMT = 64 * kMW;
 // 0.813 -> 0.790-0.797 ms (stories15M T=256, same-box A/B).
 constexpr int kAttnRows = 8;
 static_assert(kAttnRows % kMW == 0 && kAttnRows <= 16, "rows per wave");
+
+constexpr int kAttnChunks = 2;   // 256 positions each
+// Where these kernels run: T <= 512 (a row's softmax in registers, a tile's
+// rows in 64 KB of LDS) and few enough rows that the launches they save
+// count for more than the T x T arrays they move.  Whole steps, us, here /
+// tiled: 6 heads x 256 592 / 651, 8 x 256 484 / 520, 6 x 384 781 / 783,
+// 12 x 256 527 / 498, 8 x 384 785 / 738, 6 x 512 909 / 877.
+inline bool lds_rows_attention(int T, int heads, int head_dim) {
+    return head_dim % 16 == 0 && T <= 256 * kAttnChunks && (long)T * heads <= 2400;
+}
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 
@@ -773,10 +624,9 @@ struct AttnWsum {
 };
 
 // A row's first kw (a multiple of 16) LDS entries, 4 consecutive per lane
-// in up to kAttnChunks chunks of 256 (T <= 1024): x[c] holds keys
+// in up to kAttnChunks chunks of 256 (T <= 512): x[c] holds keys
 // 256c + 4*lane + (0..3); chunks at or past kw read as zeros.  Addresses
 // are clamped into the row so that every lane's read stays inside it.
-constexpr int kAttnChunks = 4;
 __device__ __forceinline__ void row_chunks(const float *row, int kw, float4 (&x)[kAttnChunks]) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
@@ -1055,27 +905,6 @@ __global__ __launch_bounds__(kMT) void k_attn_bwd_cols_mfma(const float *qkv, co
     });
 }
 
-// rope_backward (pt_backward_ops.c:52-69) of d_q, d_k, packed with d_v into
-// the fused [dq | dk | dv] row used by the QKV GEMMs.
-__global__ void k_rope_bwd_pack(const float *d_q, const float *d_k, const float *d_v, float *d_qkv, int R, int D,
-                                int KV, int QS, int hd) {
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int pairs = D / 2;
-    if (idx >= (long)R * pairs) return;
-    const int t = (int)(idx / pairs), i = 2 * (int)(idx % pairs);
-    float c, s;
-    d_rope_cs(i, hd, t, &c, &s);
-    const float q0 = d_q[(long)t * D + i], q1 = d_q[(long)t * D + i + 1];
-    const float k0 = d_k[(long)t * KV + i], k1 = d_k[(long)t * KV + i + 1];
-    float *o = d_qkv + (long)t * QS;
-    o[i] = q0 * c + q1 * s;
-    o[i + 1] = -q0 * s + q1 * c;
-    o[D + i] = k0 * c + k1 * s;
-    o[D + i + 1] = -k0 * s + k1 * c;
-    o[D + KV + i] = d_v[(long)t * KV + i];
-    o[D + KV + i + 1] = d_v[(long)t * KV + i + 1];
-}
-
 // embedding_backward (pt_backward_ops.c:90-95) in the reference's order:
 // the block of the first position holding a token accumulates, per column,
 // every position with that token in ascending t.  One pass over tok marks
@@ -1164,21 +993,25 @@ int train_create(ptmi_model *m) {
     TrainState *ts = new TrainState();
     const size_t T = m->max_T, D = c.dim, H = c.hidden, L = c.n_layers, V = c.vocab, KV = c.kv_dim;
     const size_t NH = c.n_heads, QS = D + 2 * KV;
+    // the longest T whose attention keeps its score rows
+    size_t TA = T;
+    while (TA > 0 && !lds_rows_attention((int)TA, (int)NH, c.head_dim)) TA--;
     ts->T_max = (int)T;
     ts->ws_floats = (size_t)8 << 20;
     size_t sizes[] = {
-        (L + 1) * T * D, L * T * D, L * T * D, L * T * QS, L * NH * T * T, L * T * D, L * T * D, L * T * 2 * H,
+        (L + 1) * T * D, L * T * D, L * T * D, L * T * QS, L * NH * TA * TA, L * T * D, L * T * D, L * T * 2 * H,
         T * H, T * D, T * V,                                   // forward
         m->res->mem_floats,                                    // grads
-        (2 * L + 2) * T * D, (2 * L + 1) * T * D, T * H, L * T * 2 * H, L * T * H, T * D, T * D, T * KV, T * KV,
-        L * T * QS, NH * T * T, (2 * L + 1) * T, T, 64, ts->ws_floats, T, 1,
-        (gemm_group_desc_bytes(4 * (int)L + 1) + 3) / 4, (sizeof(NormDw) * (2 * L + 1) + 3) / 4, (V + 31) / 32};
+        (2 * L + 2) * T * D, (2 * L + 1) * T * D, T * H, L * T * 2 * H, L * T * H, T * D,
+        L * T * QS, NH * TA * TA, (2 * L + 1) * T, T, 64, ts->ws_floats, T, 1,
+        (gemm_group_desc_bytes(4 * (int)L + 1) + 3) / 4, (sizeof(NormDw) * (2 * L + 1) + 3) / 4, (V + 31) / 32,
+        2 * L * NH * align_up(T, 16), NH * align_up(T, 16)};
     float *dw_desc = nullptr;
     float **dst[] = {&ts->res, &ts->res_att, &ts->xb_att, &ts->qkv, &ts->att, &ts->att_out, &ts->xb_ffn, &ts->h13,
                      &ts->sh, &ts->x_final, &ts->logits, &ts->gmem, &ts->d_res, &ts->d_xb, &ts->d_sh, &ts->d_h13,
-                     &ts->shb, &ts->d_aout, &ts->d_q, &ts->d_k, &ts->d_v, &ts->d_qkv, &ts->ds, &ts->row_inv,
+                     &ts->shb, &ts->d_aout, &ts->d_qkv, &ts->ds, &ts->row_inv,
                      &ts->row_loss, &ts->loss, &ts->ws, (float **)&ts->tok, &ts->lr, &dw_desc, &ts->nd_desc,
-                     (float **)&ts->tok_bits};
+                     (float **)&ts->tok_bits, &ts->stat, &ts->delta};
     const int nbuf = (int)(sizeof(sizes) / sizeof(sizes[0]));
     size_t total = 0;
     for (int i = 0; i < nbuf; i++) total += align_up(sizes[i], 64);
@@ -1319,7 +1152,7 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     const Resident *r = m->res;
     const Config &c = m->c;
     const int D = c.dim, H = c.hidden, L = c.n_layers, V = c.vocab, KV = c.kv_dim, NH = c.n_heads, hd = c.head_dim;
-    const int QS = D + 2 * KV, R = T - 1, kv_mul = c.n_heads / c.n_kv_heads;
+    const int QS = D + 2 * KV, R = T - 1;
     const float scale = host_scale(hd);
     const long TD = (long)T * D;
     auto G = [&](const float *p) { return ts->gmem + (p - r->mem); };   // grad of a weight tensor
@@ -1329,15 +1162,8 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     do { if (tr && (st = tr->begin(name_, cat_, layer_))) return st; } while (0)
 #define SPAN_END() \
     do { if (tr && (st = tr->end())) return st; } while (0)
-    const size_t att_lds = (size_t)T * sizeof(float);
-    // G lanes per head row: the smallest of 8/16/32 with 4*G >= head_dim
-    const int hd4 = hd / 4;
-    auto attn_fwd = hd4 <= 8 ? k_attn_fwd<8> : hd4 <= 16 ? k_attn_fwd<16> : k_attn_fwd<32>;
-    auto attn_bwd_rows = hd4 <= 8 ? k_attn_bwd_rows<8> : hd4 <= 16 ? k_attn_bwd_rows<16> : k_attn_bwd_rows<32>;
-    auto attn_bwd_cols = hd4 <= 8 ? k_attn_bwd_cols<8> : hd4 <= 16 ? k_attn_bwd_cols<16> : k_attn_bwd_cols<32>;
-    // The matrix-core attention kernels when head_dim is a multiple of 16 (up
-    // to 128), a row fits the softmax's registers and the LDS fits in 64 KB;
-    // otherwise the per-position ones.
+    // Attention: whole score rows in LDS for short and few rows (its backward
+    // also saves the launch of the Wo product), else the tiled kernels.
     using MfFwd = void (*)(const float *, float *, float *, int, int, int, float, int);
     using MfRows = void (*)(const float *, const float *, float *, const float *, const float *, float *, float *, int,
                             int, int, int, float,
@@ -1354,8 +1180,10 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     const int HQ = hd / 16, pitch = (T + 15) / 16 * 16 + 4;
     const size_t mf_lds = std::max<size_t>((size_t)16 * pitch, (size_t)kMW * 16 * hd) * sizeof(float);
     const size_t mc_lds = (size_t)kMW * 16 * hd * sizeof(float);
-    const bool mfma_attn =
-        hd % 16 == 0 && HQ >= 1 && HQ <= 8 && KV == D && T <= 256 * kAttnChunks && mf_lds <= 65536;
+    const bool row_attn = lds_rows_attention(T, NH, hd);
+    const long stat_ld = align_up(T, 16);
+    auto row_max = [&](int l) { return ts->stat + (long)l * NH * stat_ld; };
+    auto row_inv = [&](int l) { return ts->stat + (long)(L + l) * NH * stat_ld; };
 
     // pt_zero_grads (pt_train.c:425-427) is implicit: every gradient below is
     // written, not accumulated, by the one kernel that produces it (0 + v is
@@ -1432,12 +1260,13 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
             return st;
         SPAN_END();
         SPAN("attention", "fwd", l);
-        if (mfma_attn)
+        if (row_attn) {
             hipLaunchKernelGGL(mf_fwd[HQ - 1], dim3((T + kAttnRows - 1) / kAttnRows, NH), dim3(kMT), mf_lds, s, qkv, att,
                                ao, T, D, QS, scale, pitch);
-        else
-            hipLaunchKernelGGL(attn_fwd, dim3(T, NH), dim3(kAttnThreads), att_lds, s, qkv, att, ao, T, D, QS, KV, hd,
-                               kv_mul, scale);
+        } else {
+            const AttnFwdArgs fa = {qkv, QS, qkv + D, qkv + 2 * D, QS, ao, D, row_max(l), row_inv(l), stat_ld, T, 0, hd, scale};
+            if ((st = launch_attn_fwd(fa, NH, s))) return st;
+        }
         // residual: rmid = rin + att_out . Wo^T (inside the attention span,
         // as pt_train.c:222-258 keeps the Wo matvecs)
         if ((st = gemm(s, ts, 2, ao, D, r->wo + (long)l * D * D, D, rmid, D, T, D, D, 1, rin))) return st;
@@ -1534,26 +1363,23 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
         if ((st = gemm(s, ts, 0, dh13, 2 * H, w13, D, dxb(v), D, R, D, 2 * H, 0, nullptr, &pk))) return st;
         norm_bwd(rmid, r->rms_ffn + (long)l * D);
         SPAN_END();
-        // Wo: d_aout = d_res . Wo, inside the matrix-core attention rows
+        // Wo: d_aout = d_res . Wo, inside the LDS-row attention's rows
         // kernel when D splits over its waves in whole MFMA k steps
-        const bool wo_fused = mfma_attn && D % (4 * kMW) == 0;
+        const bool wo_fused = row_attn && D % (4 * kMW) == 0;
         SPAN("wo", "bwd", l);
         if (!wo_fused && (st = gemm(s, ts, 0, dres(v), D, wo, D, ts->d_aout, D, R, D, D, 0))) return st;
         SPAN_END();
         // attention
         SPAN("attention", "bwd", l);
-        if (mfma_attn) {
+        if (row_attn) {
             hipLaunchKernelGGL(mf_rows[HQ - 1], dim3((R + kAttnRows - 1) / kAttnRows, NH), dim3(kMT), mf_lds, s, qkv,
                                att, ts->d_aout, wo_fused ? dres(v) : nullptr, wo, ts->ds, dqkv, T, R, D, QS, scale, pitch);
             hipLaunchKernelGGL(mf_cols[HQ - 1], dim3((R + 15) / 16, NH), dim3(kMT), mc_lds, s, qkv, att, ts->ds,
                                ts->d_aout, dqkv, T, R, D, QS);
         } else {
-            hipLaunchKernelGGL(attn_bwd_rows, dim3(R, NH), dim3(kAttnThreads), att_lds, s, qkv, att, ts->d_aout, ts->ds,
-                               ts->d_q, T, D, QS, KV, hd, kv_mul, scale);
-            hipLaunchKernelGGL(attn_bwd_cols, dim3(R, NH), dim3(kAttnThreads), 2 * att_lds, s, qkv, att, ts->ds,
-                               ts->d_aout, ts->d_k, ts->d_v, T, R, D, QS, KV, hd, kv_mul);
-            hipLaunchKernelGGL(k_rope_bwd_pack, dim3(blocks_for((long)R * D / 2, 256)), dim3(256), 0, s, ts->d_q,
-                               ts->d_k, ts->d_v, dqkv, R, D, KV, QS, hd);
+            const AttnBwdArgs ba = {qkv, QS, ts->att_out + l * TD, ts->d_aout, row_max(l), row_inv(l), ts->delta, stat_ld,
+                                    dqkv, R, D, hd, scale};
+            if ((st = launch_attn_bwd(ba, NH, s))) return st;
         }
         PTMI_HIP(hipGetLastError());
         SPAN_END();

@@ -36,9 +36,9 @@ def tensor_slices(cfg):
     return out, o
 
 
-# head_dim 16 / 32 / 32 / 80 / 128 take the matrix-core attention kernels
-# (T = 16, 64, 2, 24, 144: whole, ragged and single 16-row tiles); head_dim
-# 24 and 36 (not multiples of 16) the per-position ones.  Vocab 1501 and 301
+# head_dim 16 / 32 / 32 / 80 / 128 take the attention kernels with score rows
+# in LDS (T = 16, 64, 2, 24, 144: whole, ragged and single 16-row tiles);
+# head_dim 24 and 36 (not multiples of 16) the tiled ones.  Vocab 1501 and 301
 # exercise the loss kernel's scalar tail (vocab % 4 != 0); dim 2304 the
 # block-per-row RMSNorm kernels (dim > 2048).
 @pytest.mark.parametrize("cfg,T", [((64, 160, 2, 4, 4, 512, 32), 16), ((96, 256, 1, 3, 3, 1000, 64), 64),
@@ -147,6 +147,16 @@ def test_steps_with_changing_tokens_match_oracle(untied):
         assert np.linalg.norm(ua - ub) / np.linalg.norm(ub) < 1e-3, name
     m.close()
     om.close()
+
+
+@pytest.mark.parametrize("cfg,T", [((576, 64, 1, 36, 36, 64, 320), 317), ((128, 64, 2, 8, 8, 64, 320), 305),
+                                   ((128, 64, 1, 1, 1, 64, 520), 513), ((16, 64, 1, 4, 4, 64, 40), 33),
+                                   ((72, 64, 1, 2, 2, 64, 40), 2), ((520, 64, 1, 10, 10, 64, 260), 257)])
+def test_tiled_attention_step_matches_oracle(cfg, T):
+    """Shapes whose attention is tiled: two tiles per block with a ragged last
+    one, one tile, head_dim 128 on four waves, and head_dims that are no
+    multiple of 16 (4, 36, 52), one key and one row included."""
+    check_one_step(cfg, T)
 
 
 def test_graph_and_eager_steps_give_the_same_bits(monkeypatch):
