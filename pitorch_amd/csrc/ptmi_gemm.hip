@@ -290,6 +290,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
     static_assert(NORM == 0 || (!AT && TM == 32 && VEC && EA == 4), "fused norm: NT, 32-row float4 A tiles");
     __shared__ float As[2][BK][TM];
     __shared__ float Bs[2][BK][TN];
+constexpr int kChains = BK / 4;
+// acc[0] = the sum of the 8 partial sums, pairwise
+__device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
+#pragma unroll
+    for (int h = kChains / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int c = 0; c < h; c++) acc[c][0][0] += acc[c + h][0][0];
+}
+
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int li = lane & 15, lk = lane >> 4;
@@ -297,11 +306,19 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
     const int kend = min(g.K, kb + g.k_per_split);
     const int nk = kb < kend ? (kend - kb + BK - 1) / BK : 0;
 
-    floatx4 acc[FM][FN];
+    // One 16x16 block per wave: the 8 MFMAs of a K step go to 8 sums, added
+    // pairwise at the end, so each is rounded an eighth as often (64x768x288
+    // and its gradients: 3.0e-7 -> 1.2e-7 from 64-bit sums, 17.3 -> 16.8 us).
+    // Not TN: the 32 registers cost the grouped weight gradients occupancy
+    // (64 steps of stories15M, T=256: 50.0 -> 52.8 ms).
+    constexpr int NC = FM * FN == 1 && !AT ? kChains : 1;
+    floatx4 acc[NC][FM][FN];
 #pragma unroll
-    for (int i = 0; i < FM; i++)
+    for (int c = 0; c < NC; c++)
 #pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) acc[c][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     // P K tiles in flight in a register ring (tile t in slot t % P); the
     // loop is unrolled by P so every slot index is a compile-time constant.
@@ -387,7 +404,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
             for (int i = 0; i < FM; i++)
 #pragma unroll
                 for (int j = 0; j < FN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c][i], b[c][j], acc[i][j], 0, 0, 0);
+                    acc[kk / 4 % NC][i][j] =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(a[c][i], b[c][j], acc[kk / 4 % NC][i][j], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -430,9 +448,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
         if (tid % (BK / EA) == 0) n_inv[tid / (BK / EA)] = 1.0f / d_sqrtf(nss / (float)g.K + 1e-5f);
         __syncthreads();
         norm_rows_out<NORM, TM>(g, m0, n0 / TN, (g.N + TN - 1) / TN, n_inv);
-        gemm_store<EPI, FM, FN>(g, acc, m0 + wm * (TM / 2), n0 + wn * (TN / 2), z, li, lk, n_inv, m0);
+        gemm_store<EPI, FM, FN>(g, acc[0], m0 + wm * (TM / 2), n0 + wn * (TN / 2), z, li, lk, n_inv, m0);
+    if constexpr (NC > 1) sum_chains(acc);
     } else {
-        gemm_store<EPI, FM, FN>(g, acc, m0 + wm * (TM / 2), n0 + wn * (TN / 2), z, li, lk);
+        gemm_store<EPI, FM, FN>(g, acc[0], m0 + wm * (TM / 2), n0 + wn * (TN / 2), z, li, lk);
     }
 }
 
@@ -641,7 +660,9 @@ __device__ __forceinline__ void gemm_tile_panel(const GemmArgs &g, int m0, int n
         dl_issue<false, TM, NW>(g.A, g.lda, g.M, m0, kb + t * BK, kend, st, junk, wave, lane);
         dl_issue<BKM, TN, NW>(g.B, g.ldb, g.N, n0, kb + t * BK, kend, st + TM * BK, junk, wave, lane);
     }
-    floatx4 acc[1][1] = {{floatx4{0.f, 0.f, 0.f, 0.f}}};
+    floatx4 acc[kChains][1][1];                                     // as gemm_tile's
+#pragma unroll
+    for (int c = 0; c < kChains; c++) acc[c][0][0] = floatx4{0.f, 0.f, 0.f, 0.f};
     const int ia = wm * 16 + li, ib = wn * 16 + li;
     // step s, unrolled (each wait takes a constant count)
     auto step = [&](auto sc) {
@@ -670,11 +691,13 @@ __device__ __forceinline__ void gemm_tile_panel(const GemmArgs &g, int m0, int n
             for (int q = 0; q < 2; q++)
 #pragma unroll
                 for (int u = 0; u < 4; u++)
-                    acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][u], b[q][u], acc[0][0], 0, 0, 0);
+                    acc[4 * q + u][0][0] =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][u], b[q][u], acc[4 * q + u][0][0], 0, 0, 0);
         }
     };
     unrolled(step, std::make_integer_sequence<int, NSK>{});
-    gemm_store<EPI, 1, 1>(g, acc, m0 + wm * 16, n0 + wn * 16, z, li, lk);
+    sum_chains(acc);
+    gemm_store<EPI, 1, 1>(g, acc[0], m0 + wm * 16, n0 + wn * 16, z, li, lk);
 }
 
 // ── fp32 products on the bf16 matrix cores ───────────────────────────────
