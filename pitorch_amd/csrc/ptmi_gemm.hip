@@ -281,15 +281,6 @@ __device__ __forceinline__ void norm_rows_out(const GemmArgs &g, int m0, int j, 
     }
 }
 
-// One TMxTN output tile of g at (m0, n0) over K range split z.  The LDS
-// tiles use the swizzled layout of lds_col.
-template <bool AT, bool BT, int TM, int TN, int P, bool VEC, int EPI = GEMM_EPI_NONE, int NORM = 0>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int z) {
-    constexpr int FM = TM / 32, FN = TN / 32;          // 16x16 MFMA blocks per wave
-    constexpr int EA = TM * BK / 256, EB = TN * BK / 256;
-    static_assert(NORM == 0 || (!AT && TM == 32 && VEC && EA == 4), "fused norm: NT, 32-row float4 A tiles");
-    __shared__ float As[2][BK][TM];
-    __shared__ float Bs[2][BK][TN];
 constexpr int kChains = BK / 4;
 // acc[0] = the sum of the 8 partial sums, pairwise
 __device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
@@ -299,6 +290,15 @@ __device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
         for (int c = 0; c < h; c++) acc[c][0][0] += acc[c + h][0][0];
 }
 
+// One TMxTN output tile of g at (m0, n0) over K range split z.  The LDS
+// tiles use the swizzled layout of lds_col.
+template <bool AT, bool BT, int TM, int TN, int P, bool VEC, int EPI = GEMM_EPI_NONE, int NORM = 0>
+__device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int z) {
+    constexpr int FM = TM / 32, FN = TN / 32;          // 16x16 MFMA blocks per wave
+    constexpr int EA = TM * BK / 256, EB = TN * BK / 256;
+    static_assert(NORM == 0 || (!AT && TM == 32 && VEC && EA == 4), "fused norm: NT, 32-row float4 A tiles");
+    __shared__ float As[2][BK][TM];
+    __shared__ float Bs[2][BK][TN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int li = lane & 15, lk = lane >> 4;
@@ -308,7 +308,7 @@ __device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
 
     // One 16x16 block per wave: the 8 MFMAs of a K step go to 8 sums, added
     // pairwise at the end, so each is rounded an eighth as often (64x768x288
-    // and its gradients: 3.0e-7 -> 1.2e-7 from 64-bit sums, 17.3 -> 16.8 us).
+    // and its gradients: 3.0e-7 -> 1.2e-7 from 64-bit sums, 17 us as before).
     // Not TN: the 32 registers cost the grouped weight gradients occupancy
     // (64 steps of stories15M, T=256: 50.0 -> 52.8 ms).
     constexpr int NC = FM * FN == 1 && !AT ? kChains : 1;
@@ -440,6 +440,7 @@ __device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
         }
     }
 
+    if constexpr (NC > 1) sum_chains(acc);
     if constexpr (NORM != 0) {
         // 1/rms of the block's rows (the standalone kernel's formula); every
         // N tile's block stores its share of the rows and normalized rows
@@ -449,7 +450,6 @@ __device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
         __syncthreads();
         norm_rows_out<NORM, TM>(g, m0, n0 / TN, (g.N + TN - 1) / TN, n_inv);
         gemm_store<EPI, FM, FN>(g, acc[0], m0 + wm * (TM / 2), n0 + wn * (TN / 2), z, li, lk, n_inv, m0);
-    if constexpr (NC > 1) sum_chains(acc);
     } else {
         gemm_store<EPI, FM, FN>(g, acc[0], m0 + wm * (TM / 2), n0 + wn * (TN / 2), z, li, lk);
     }
