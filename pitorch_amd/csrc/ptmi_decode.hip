@@ -582,9 +582,10 @@ int ptmi_model_create(const void *blob, size_t bytes, int max_T, ptmi_model_t **
         }
         memcpy(m->prefetch_plan, pp, 8);
     }
-    if ((st = decode_step_create(m)) || (!m->eager && (st = build_graph(m))) ||
+    if ((st = decode_step_create(m)) || (st = prefill_create(m)) || (!m->eager && (st = build_graph(m))) ||
         (max_T > 0 && (st = train_create(m)))) {
         train_destroy(m);
+        prefill_destroy(m);
         decode_step_destroy(m);
         if (m->exec) (void)hipGraphExecDestroy(m->exec);
         if (m->graph) (void)hipGraphDestroy(m->graph);
@@ -608,6 +609,7 @@ void ptmi_model_destroy(ptmi_model_t *m) {
     if (m->exec_k) (void)hipGraphExecDestroy(m->exec_k);
     if (m->graph_k) (void)hipGraphDestroy(m->graph_k);
     decode_step_destroy(m);
+    prefill_destroy(m);
     (void)hipFree(m->mem);
     release_blob(m->res);
     delete m;
@@ -672,9 +674,15 @@ int ptmi_model_generate(ptmi_model_t *m, const int *prompt, int n_prompt, int ma
     int st;
     if ((st = zero_kv(m))) return st;
     PTMI_HIP(hipMemcpyAsync(m->prompt, prompt, (size_t)n_prompt * sizeof(int), hipMemcpyHostToDevice, s));
-    if ((st = set_ctl(m, prompt[0], 0, n_prompt))) return st;
-    if ((st = launch_steps(m, s, max_tokens))) return st;
-    PTMI_HIP(hipMemcpyAsync(out, m->out_tokens, (size_t)max_tokens * sizeof(int), hipMemcpyDeviceToHost, s));
+    // The positions whose next token the prompt forces need only their keys
+    // and values: one pass over the weights for all of them.
+    const int n_pre = prefill_positions(m, n_prompt, max_tokens);
+    if (n_pre > 0 && (st = enqueue_prefill(m, n_pre, s))) return st;
+    for (int i = 0; i < n_pre; i++) out[i] = prompt[i + 1];
+    if ((st = set_ctl(m, prompt[n_pre], n_pre, n_prompt))) return st;
+    if ((st = launch_steps(m, s, max_tokens - n_pre))) return st;
+    PTMI_HIP(hipMemcpyAsync(out + n_pre, m->out_tokens + n_pre, (size_t)(max_tokens - n_pre) * sizeof(int),
+                            hipMemcpyDeviceToHost, s));
     DecodeCtl h;
     PTMI_HIP(hipMemcpyAsync(&h, m->ctl, sizeof(h), hipMemcpyDeviceToHost, s));
     PTMI_HIP(hipStreamSynchronize(s));

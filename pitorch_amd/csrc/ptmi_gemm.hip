@@ -163,14 +163,22 @@ __device__ __forceinline__ void store_tile(float (*S)[R], int tid, const float (
 template <int EPI>
 __device__ __forceinline__ void store_elem(const GemmArgs &g, float v, int m, int n, int z, float lrv) {
     if constexpr (EPI == GEMM_EPI_ROPE) {
-        // RoPE of the q and k columns at position m (pt_ops.c:33-49;
+        // RoPE of the q and k columns at the row's position (pt_ops.c:33-49;
         // training forward pt_train.c:217)
         const float pv = dpp_xor1(v);
-        if (n < 2 * g.epi.rope_dim) {
-            const int ip = (n < g.epi.rope_dim ? n : n - g.epi.rope_dim) & ~1;
+        const int D = g.epi.rope_dim, col = n + g.epi.col0;
+        if (col < 2 * D) {
+            const int ip = (col < D ? col : col - D) & ~1;
             float c, sn;
-            d_rope_cs(ip, g.epi.head_dim, m, &c, &sn);
+            d_rope_cs(ip, g.epi.head_dim, g.epi.pos0 + m, &c, &sn);
             v = (n & 1) ? pv * sn + v * c : v * c - pv * sn;
+        }
+        if (g.epi.out && col >= D) {                             // k and v to the caches
+            if (n < g.N && m < g.M) {
+                if (col < 2 * D) g.epi.out[(long)m * g.epi.ld + (col - D)] = v;
+                else g.epi.out2[(long)m * g.epi.ld + (col - 2 * D)] = v;
+            }
+            return;
         }
     } else if constexpr (EPI == GEMM_EPI_SWIGLU) {
         // columns (2i, 2i+1) = (h1, h3): out[m][i] = (h1*sigmoid(h1))*h3,
@@ -180,6 +188,7 @@ __device__ __forceinline__ void store_elem(const GemmArgs &g, float v, int m, in
             const float sig = 1.0f / (1.0f + d_expf(-v));
             g.epi.out[(long)m * g.epi.ld + (n >> 1)] = (v * sig) * pv;
         }
+        if (g.epi.only_out) return;
     }
     if (n >= g.N || m >= g.M) return;
     if constexpr (EPI == GEMM_EPI_SWIGLU_BWD) {
@@ -1331,7 +1340,9 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
         return set_error(PTMI_ERR_ARG, "gemm: the fused norm does not fit this GEMM");
     if (ek == GEMM_EPI_SWIGLU_BWD ? (op != 0 || !epi->out || !epi->out2 || !epi->aux)
                                   : ek != GEMM_EPI_NONE && (op != 2 || N % 2 || (ek == GEMM_EPI_SWIGLU && !epi->out) ||
-                                                            (ek == GEMM_EPI_ROPE && (epi->rope_dim % 2 || epi->head_dim <= 0))))
+                                                            (ek == GEMM_EPI_ROPE &&
+                                                             (epi->rope_dim % 2 || epi->head_dim <= 0 || epi->col0 % 2 ||
+                                                              (epi->out && (!epi->out2 || N + epi->col0 != 3 * epi->rope_dim))))))
         return set_error(PTMI_ERR_ARG, "gemm: fused epilogue %d does not fit this GEMM", ek);
     if (M <= 0 || N <= 0 || K <= 0) return set_error(PTMI_ERR_ARG, "gemm: M=%d N=%d K=%d", M, N, K);
     if (!A || !B || !C) return set_error(PTMI_ERR_ARG, "gemm: null operand");

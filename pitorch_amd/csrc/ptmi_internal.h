@@ -341,23 +341,27 @@ __device__ __forceinline__ float sum_splits(const float *parts, int splits, long
 }
 
 // Element-wise epilogues fused into an NT GEMM (whole K, no split):
-//  GEMM_EPI_ROPE: RoPE at position m on columns [0, 2*rope_dim) (q then k),
-//    applied to C in place;
+//  GEMM_EPI_ROPE: RoPE at position pos0 + m on columns [0, 2*rope_dim) (q then
+//    k) of the [q | k | v] columns, of which C's column n is number col0 + n,
+//    applied to C in place.  With `out` the k and v columns go to
+//    out[m*ld + i] and out2[m*ld + i] (i < rope_dim) and not to C;
 //  GEMM_EPI_SWIGLU: C columns (2i, 2i+1) hold (h1, h3); also writes
-//    out[m*ld + i] = (h1*sigmoid(h1))*h3.
+//    out[m*ld + i] = (h1*sigmoid(h1))*h3, and with only_out just that.
 //  GEMM_EPI_SWIGLU_BWD (NN GEMM): C[m][i] is d_sh; with (h1, h3) =
 //    aux[m*aux_ld + 2i + {0,1}] it writes d_h1, d_h3 to out[m*ld + 2i + {0,1}]
 //    and silu(h1)*h3 to out2[m*ld2 + i]; C itself is not stored.
 enum { GEMM_EPI_NONE = 0, GEMM_EPI_ROPE = 1, GEMM_EPI_SWIGLU = 2, GEMM_EPI_SWIGLU_BWD = 3 };
 struct GemmEpi {
     int kind;
-    float *out;            // SWIGLU / SWIGLU_BWD output
+    float *out;            // SWIGLU / SWIGLU_BWD output; ROPE: k rows (null: k and v stay in C)
     long ld;               // its row stride
     int rope_dim, head_dim;
-    float *out2;           // SWIGLU_BWD: recomputed silu(h1)*h3
+    float *out2;           // SWIGLU_BWD: recomputed silu(h1)*h3; ROPE with out: v rows
     long ld2;
     const float *aux;      // SWIGLU_BWD: the forward's (h1, h3) pairs
     long aux_ld;
+    int pos0, col0;        // ROPE: position of row 0, [q | k | v] column of column 0
+    int only_out;          // SWIGLU: C is not stored
 };
 
 // RMSNorm (pt_ops.c:5-12) fused into the A operand of an NT GEMM with a

@@ -124,10 +124,10 @@ __device__ __forceinline__ float dot4(float4 a, float4 b) { return a.x * b.x + a
 
 // ── forward kernels ──────────────────────────────────────────────────────
 
-// (also marks tok[t] in tok_bits for t < R)
+// (with tok_bits also marks tok[t] there for t < R)
 __global__ void k_embed_rows(const int *tok, const float *emb, float *out, int D, unsigned *tok_bits, int R) {
     const int t = blockIdx.x;                                    // pt_train.c:189-191
-    if (threadIdx.x == 0 && t < R) atomicOr(&tok_bits[tok[t] >> 5], 1u << (tok[t] & 31));
+    if (tok_bits && threadIdx.x == 0 && t < R) atomicOr(&tok_bits[tok[t] >> 5], 1u << (tok[t] & 31));
     const float *src = emb + (long)tok[t] * D;
     for (int i = threadIdx.x; i < D; i += blockDim.x) out[(long)t * D + i] = src[i];
 }
@@ -348,8 +348,8 @@ __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(
 
 // k_rmsnorm_rows, one wave per row (rmsnorm, pt_ops.c:5-12).
 // With tok != nullptr the row is first gathered from the embedding table,
-// in[row] = emb[tok[row]] (pt_train.c:189-191), and stored; rows < rows-1
-// also mark their token in tok_bits.
+// in[row] = emb[tok[row]] (pt_train.c:189-191), and stored; with tok_bits
+// rows < rows-1 also mark their token there.
 template <int NV>
 __global__ __launch_bounds__(256) void k_rmsnorm_rows_w(float *in, const float *w, float *out, int rows, int D,
                                                        SplitK pk, const float *cin, const int *tok, const float *emb,
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_w(float *in, const float *
     for (int v = 0; v < NV; v++) wv[v] = w4[min(lane + 64 * v, d4 - 1)];
     if (tok) {                                                   // uniform
         const int tk = tok[row];
-        if (lane == 0 && row < rows - 1) atomicOr(&tok_bits[tk >> 5], 1u << (tk & 31));
+        if (tok_bits && lane == 0 && row < rows - 1) atomicOr(&tok_bits[tk >> 5], 1u << (tk & 31));
         const float4 *e4 = reinterpret_cast<const float4 *>(emb) + (long)tk * d4;
 #pragma unroll
         for (int v = 0; v < NV; v++) {
@@ -986,6 +986,23 @@ float host_scale(int head_dim) {   // 1/pt_sqrtf(hd), pt_train.c:182
 
 }  // namespace
 
+// One wave per row when D % 4 == 0 and D <= 2048, else one block per row.
+void launch_rmsnorm_rows(float *in, const float *w, float *out, int rows, int D, const SplitK &pk, const float *cin,
+                         const int *tok, const float *emb, unsigned *tok_bits, hipStream_t s) {
+    using NormFn = void (*)(float *, const float *, float *, int, int, SplitK, const float *, const int *,
+                            const float *, unsigned *);
+    static const NormFn norm_w[8] = {k_rmsnorm_rows_w<1>, k_rmsnorm_rows_w<2>, k_rmsnorm_rows_w<3>,
+                                     k_rmsnorm_rows_w<4>, k_rmsnorm_rows_w<5>, k_rmsnorm_rows_w<6>,
+                                     k_rmsnorm_rows_w<7>, k_rmsnorm_rows_w<8>};
+    const int nv = (D + 255) / 256;
+    if (D % 4 == 0 && nv <= 8) {
+        hipLaunchKernelGGL(norm_w[nv - 1], dim3(rows), dim3(64), 0, s, in, w, out, rows, D, pk, cin, tok, emb, tok_bits);
+    } else {
+        if (tok) hipLaunchKernelGGL(k_embed_rows, dim3(rows), dim3(256), 0, s, tok, emb, in, D, tok_bits, rows - 1);
+        hipLaunchKernelGGL(k_rmsnorm_rows, dim3(rows), dim3(256), 0, s, in, w, out, D, pk, cin);
+    }
+}
+
 int train_create(ptmi_model *m) {
     const Config &c = m->c;
     if (c.kv_dim != c.dim)
@@ -1191,14 +1208,8 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     // The one accumulation is the embedding's: with the classifier tied to
     // it, the classifier's dW (written first) is its starting value;
     // untied, its rows are cleared here.
-    // RMSNorm rows: one wave per row when D % 4 == 0 and D <= 2048, else one
-    // block per row.
-    using NormFn = void (*)(float *, const float *, float *, int, int, SplitK, const float *, const int *,
-                            const float *, unsigned *);
+    // RMSNorm rows: as launch_rmsnorm_rows.
     using NormBwdFn = void (*)(float *, const float *, float *, const float *, const float *, float *, int, int, SplitK);
-    static const NormFn norm_w[8] = {k_rmsnorm_rows_w<1>, k_rmsnorm_rows_w<2>, k_rmsnorm_rows_w<3>,
-                                     k_rmsnorm_rows_w<4>, k_rmsnorm_rows_w<5>, k_rmsnorm_rows_w<6>,
-                                     k_rmsnorm_rows_w<7>, k_rmsnorm_rows_w<8>};
     static const NormBwdFn norm_bwd_w[8] = {k_rmsnorm_bwd_rows_w<1>, k_rmsnorm_bwd_rows_w<2>, k_rmsnorm_bwd_rows_w<3>,
                                             k_rmsnorm_bwd_rows_w<4>, k_rmsnorm_bwd_rows_w<5>, k_rmsnorm_bwd_rows_w<6>,
                                             k_rmsnorm_bwd_rows_w<7>, k_rmsnorm_bwd_rows_w<8>};
@@ -1206,14 +1217,7 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     const bool wave_norm = D % 4 == 0 && nv <= 8;
     // embed: gather the rows from the embedding table first (layer 0)
     auto norm_fwd = [&](float *in, const float *w, float *out, SplitK pk, const float *cin, bool embed) {
-        if (wave_norm) {
-            hipLaunchKernelGGL(norm_w[nv - 1], dim3(T), dim3(64), 0, s, in, w, out, T, D, pk, cin,
-                               embed ? ts->tok : nullptr, r->emb, ts->tok_bits);
-        } else {
-            if (embed) hipLaunchKernelGGL(k_embed_rows, dim3(T), dim3(256), 0, s, ts->tok, r->emb, in, D, ts->tok_bits,
-                                          T - 1);
-            hipLaunchKernelGGL(k_rmsnorm_rows, dim3(T), dim3(256), 0, s, in, w, out, D, pk, cin);
-        }
+        launch_rmsnorm_rows(in, w, out, T, D, pk, cin, embed ? ts->tok : nullptr, r->emb, ts->tok_bits, s);
     };
     // RMSNorm then an NT GEMM with a fused epilogue, C = epi(rmsnorm(x) . W^T):
     // the norm runs inside the GEMM's A loads when launch_gemm can fuse it

@@ -1,0 +1,58 @@
+"""GPU: ptmi_model_generate's prompt pass (all forced positions at once)
+against the oracle's token-by-token run (pt_text.c:344-350).
+
+The last position's logits attend to every cached key and value, so they
+check the caches of all prompt positions; one more forward_step checks that
+the model goes on from them.  Tolerance: that of the decode step against the
+oracle (1e-5 of max |logit|; only the orders of the sums differ).
+"""
+import numpy as np
+import pytest
+
+import pitorch_amd as pa
+from tests._oracle import OracleModel
+
+pytestmark = pytest.mark.gpu
+
+SMALL = (64, 160, 2, 4, 4, 512, 256)             # dim hidden layers heads kv_heads vocab seq_len
+PADDED_HEAD = (108, 260, 2, 3, 3, 512, 160)      # head_dim 36: no multiple of 16
+WIDE_HEAD = (256, 512, 2, 2, 2, 512, 96)         # head_dim 128
+ONE_LAYER = (96, 256, 1, 3, 3, 512, 96)          # keys and values only
+WIDE = (2304, 260, 1, 24, 24, 512, 48)           # norm rows past one wave's registers
+TWO_PASSES = (32, 64, 2, 2, 2, 512, 1200)        # more positions than one pass takes
+
+
+@pytest.mark.parametrize("cfg,n_prompt,total", [
+    *[(SMALL, n, n + 3) for n in (1, 2, 3, 4, 5, 6, 7, 9, 16, 17, 18, 33, 34, 65, 130, 253)],
+    (SMALL, 40, 40), (SMALL, 40, 25), (SMALL, 40, 4), (SMALL, 40, 1), (SMALL, 256, 256),
+    *[(PADDED_HEAD, n, n + 2) for n in (6, 31, 150)],
+    *[(WIDE_HEAD, n, n + 2) for n in (6, 50, 90)],
+    *[(ONE_LAYER, n, n + 2) for n in (6, 70)],
+    *[(WIDE, n, n + 2) for n in (6, 40)],
+    *[(TWO_PASSES, n, n + 2) for n in (1024, 1025, 1026, 1031, 1190)],
+])
+def test_prompt_pass_matches_oracle(cfg, n_prompt, total):
+    blob = pa.synth_model(cfg, 21)
+    prompt = np.array(pa.seed_tokens(n_prompt, n_prompt, cfg[5]), np.int32)
+    m, om = pa.Model(blob), OracleModel(blob.copy())
+    got = m.generate(prompt, total, stop_on_eos=False)
+    want, tok = [], int(prompt[0])
+    for pos in range(total):
+        nxt = om.forward_step(tok)
+        tok = int(prompt[pos + 1]) if pos + 1 < n_prompt else nxt
+        want.append(tok)
+    assert list(got) == want and m.pos() == total
+    for step in range(2):
+        lg, ref = m.logits(), om.logits()
+        assert np.max(np.abs(lg - ref)) <= 1e-5 * np.max(np.abs(ref)), step
+        if step or total == cfg[6]:
+            break
+        assert m.forward_step(tok) == om.forward_step(tok)
+    # a second prompt on the same model: nothing of the first is left
+    again = m.generate(prompt[::-1].copy(), total, stop_on_eos=False)
+    m2 = pa.Model(blob)
+    assert list(m2.generate(prompt[::-1].copy(), total, stop_on_eos=False)) == list(again)
+    assert np.array_equal(m.logits(), m2.logits())
+    m2.close()
+    m.close()
+    om.close()
