@@ -1199,20 +1199,35 @@ __global__ __launch_bounds__(256, 2) void k_gemm_split(GemmArgs g) {
     else gemm_tile_slice64<AK, BKM, E, EPI>(g, m * T, n * T, z);
 }
 
-// Grouped TN GEMMs (32x32 tiles, whole K): block b runs tile
-// t = xcd_tile(b) - d.tile0 of the descriptor d whose tile range holds it;
-// tiles run along N first, so neighbours share the A^T tile.  The launch
-// covers entries [i0, i1) of the table, whose tiles start at d[i0].tile0 (a
-// tile's result does not depend on the block that computes it, so a launch
-// of a sub-range gives the same bits as the whole table).
-template <int TM, int TN, bool VEC>
-__global__ __launch_bounds__(256) void k_gemm_tn_group(const GemmGroupDesc *d, int i0, int i1) {
+// Grouped TN GEMMs (whole K): block b runs tile t = xcd_tile(b) - d.tile0 of
+// the descriptor d whose tile range holds it.  The launch covers entries
+// [i0, i1) of the table, whose tiles start at d[i0].tile0 (a tile's result
+// does not depend on the block that computes it, so a launch of a sub-range
+// gives the same bits as the whole table).
+__device__ __forceinline__ const GemmGroupDesc &group_tile(const GemmGroupDesc *d, int i0, int i1, int &t) {
     const int b = d[i0].tile0 + xcd_tile(blockIdx.x, gridDim.x);
     int i = i0;
     while (i + 1 < i1 && d[i + 1].tile0 <= b) i++;
-    const GemmGroupDesc &e = d[i];
-    const int t = b - e.tile0;
+    t = b - d[i].tile0;
+    return d[i];
+}
+// 32x32 fp32 tiles; they run along N first, so neighbours share the A^T tile.
+template <int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256) void k_gemm_tn_group(const GemmGroupDesc *d, int i0, int i1) {
+    int t;
+    const GemmGroupDesc &e = group_tile(d, i0, i1, t);
     gemm_tile<true, false, TM, TN, kRing32, VEC>(e.g, (t / e.tiles_n) * TM, (t % e.tiles_n) * TN, 0);
+}
+// 64x64 tiles of bf16 products; neighbours share the tile of the larger operand.
+template <int E>
+__global__ __launch_bounds__(256, 2) void k_gemm_tn_group_split(const GemmGroupDesc *d, int i0, int i1) {
+    int t;
+    const GemmGroupDesc &e = group_tile(d, i0, i1, t);
+    const int gx = e.tiles_n, gy = (e.g.M + 63) / 64;
+    int m, n;
+    if (e.g.M > e.g.N) m = t / gx, n = t - m * gx;
+    else n = t / gy, m = t - n * gy;
+    gemm_tile_slice64<true, true, E, GEMM_EPI_NONE>(e.g, m * 64, n * 64, 0);
 }
 
 // C = (Cin +) sum_z partial[z], z ascending.
@@ -1464,10 +1479,26 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
 
 size_t gemm_group_desc_bytes(int n) { return sizeof(GemmGroupDesc) * (size_t)n; }
 
-int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host_desc, int *tiles_total,
-                          int *vec_out) {
+int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host_desc, TnGroupPlan *plan) {
     GemmGroupDesc *d = static_cast<GemmGroupDesc *>(host_desc);
-    int t = 0, vec = 1;
+    int vec = 1;
+    // Tile: the smaller estimate over all entries.  The 64 tiles' is
+    // gemm_choice's plus 4.4 us per tile for the weights' update, which the
+    // many 32x32 blocks hide behind each other's products.  Whole training
+    // steps with 32 / 64 tiles, us: stories110M T=256 3276 / 3649, T=512 4862 /
+    // 4852, T=1024 8470 / 7661; stories42M T=512 2316 / 2370; 252-wide, 7
+    // layers, T=700 1138 / 1115.
+    double us32 = 3.2, us64 = 4.0;
+    bool fits = true;
+    for (int i = 0; i < n; i++) {
+        const TnGemm &e = list[i];
+        auto blocks = [&](int T) { return (double)((e.M + T - 1) / T) * ((e.N + T - 1) / T); };
+        us32 += (e.K + BK - 1) / BK * 0.19 * blocks(32) / 256.0;
+        us64 += (7.0 + 0.65 * ((e.K + 63) / 64)) * blocks(64) / 256.0;
+        fits = fits && e.lda < kMaxSplitLd && e.ldb < kMaxSplitLd;
+    }
+    const int tile = fits && us64 < us32 ? 64 : 32;
+    int t = 0;
     for (int i = 0; i < n; i++) {
         const TnGemm &e = list[i];
         if (e.M <= 0 || e.N <= 0 || e.K <= 0 || !e.A || !e.B || !e.C || e.lda < e.M || e.ldb < e.N || e.ldc < e.N)
@@ -1479,19 +1510,24 @@ int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host
         if (e.upd && !lr) return set_error(PTMI_ERR_ARG, "grouped gemm %d: update without a learning rate", i);
         g.upd = e.upd; g.lr = lr; g.keep = e.keep;
         if (!(al16(e.A) && e.lda % 4 == 0 && e.M % 4 == 0 && al16(e.B) && e.ldb % 4 == 0 && e.N % 4 == 0)) vec = 0;
-        d[i].tiles_n = (e.N + 31) / 32;
+        d[i].tiles_n = (e.N + tile - 1) / tile;
         d[i].tile0 = t;
-        t += d[i].tiles_n * ((e.M + 31) / 32);
+        t += d[i].tiles_n * ((e.M + tile - 1) / tile);
+        if (i == 0) plan->first_tiles = t;
     }
-    *tiles_total = t;
-    *vec_out = vec;
+    plan->tiles = t;
+    plan->vec = vec;
+    plan->tile = tile;
     return PTMI_OK;
 }
 
-int launch_gemm_tn_group(const void *dev_desc, int i0, int i1, int tiles, int vec, hipStream_t s) {
+int launch_gemm_tn_group(const void *dev_desc, int i0, int i1, int tiles, const TnGroupPlan &plan, hipStream_t s) {
     if (i1 <= i0 || tiles <= 0) return PTMI_OK;
-    void (*fn)(const GemmGroupDesc *, int, int) = vec ? k_gemm_tn_group<32, 32, true> : k_gemm_tn_group<32, 32, false>;
-    hipLaunchKernelGGL(fn, dim3((unsigned)tiles), dim3(256), 0, s, static_cast<const GemmGroupDesc *>(dev_desc), i0, i1);
+    using Fn = void (*)(const GemmGroupDesc *, int, int);
+    static const Fn fns[2][2] = {{k_gemm_tn_group<32, 32, false>, k_gemm_tn_group<32, 32, true>},
+                                 {k_gemm_tn_group_split<1>, k_gemm_tn_group_split<4>}};
+    hipLaunchKernelGGL(fns[plan.tile == 64][plan.vec], dim3((unsigned)tiles), dim3(256), 0, s,
+                       static_cast<const GemmGroupDesc *>(dev_desc), i0, i1);
     PTMI_HIP(hipGetLastError());
     return PTMI_OK;
 }

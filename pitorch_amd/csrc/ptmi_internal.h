@@ -409,7 +409,7 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
 size_t gemm_workspace_floats(int op, int M, int N, int K, size_t ws_floats);
 
 // Grouped C[M,N] = A^T.B GEMMs (TN; A stored [K][M]; C written, not
-// accumulated), one launch of 32x32 tiles over all of them.  prepare fills host_desc (gemm_group_desc_bytes(n)
+// accumulated), one launch of 32x32 or 64x64 tiles over all of them.  prepare fills host_desc (gemm_group_desc_bytes(n)
 // bytes); the caller copies it to device memory for the launch.
 // upd != null: the SGD step of the weight whose gradient C is, fused into
 // the epilogue: upd[m][n] -= *lr * C[m][n] (same layout as C), except rows
@@ -424,9 +424,15 @@ struct TnGemm {
     const unsigned *keep = nullptr;
 };
 size_t gemm_group_desc_bytes(int n);
-int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host_desc, int *tiles_total, int *vec);
+struct TnGroupPlan {
+    int tile = 32;         // tile size
+    int tiles = 0;         // tiles of the whole table
+    int first_tiles = 0;   // tiles of its entry 0
+    int vec = 0;           // 16-byte rows throughout
+};
+int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host_desc, TnGroupPlan *plan);
 // Entries [i0, i1) of a prepared table, whose tiles number `tiles`.
-int launch_gemm_tn_group(const void *dev_desc, int i0, int i1, int tiles, int vec, hipStream_t s);
+int launch_gemm_tn_group(const void *dev_desc, int i0, int i1, int tiles, const TnGroupPlan &plan, hipStream_t s);
 
 // Causal attention of all heads over `rows` positions on the matrix cores
 // (head_dim a multiple of 4, at most 128; row strides and head_dim multiples

@@ -41,7 +41,8 @@ struct TrainState {
     // Descriptor tables of the two grouped launches (device; built per T).
     void *dw_desc;
     float *nd_desc;
-    int desc_T = 0, dw_tiles = 0, n_dw = 0, dw_vec = 0, dw_cls_tiles = 0;   // entry 0: the classifier
+    int desc_T = 0, n_dw = 0;   // entry 0: the classifier
+    TnGroupPlan dw_plan;
     float *ws;
     size_t ws_floats = 0;
     float *lr;                  // device copy of the step's learning rate (lr_off floats past tok)
@@ -1117,14 +1118,13 @@ int train_descriptors(ptmi_model *m, int T) {
         v++;
     }
     std::vector<char> host(gemm_group_desc_bytes((int)g.size()));
-    int tiles = 0, vec = 0, st;
-    if ((st = gemm_tn_group_prepare(g.data(), (int)g.size(), ts->lr, host.data(), &tiles, &vec))) return st;
+    TnGroupPlan plan;
+    int st;
+    if ((st = gemm_tn_group_prepare(g.data(), (int)g.size(), ts->lr, host.data(), &plan))) return st;
     PTMI_HIP(hipMemcpy(ts->dw_desc, host.data(), host.size(), hipMemcpyHostToDevice));
     PTMI_HIP(hipMemcpy(ts->nd_desc, nd.data(), nd.size() * sizeof(NormDw), hipMemcpyHostToDevice));
     ts->n_dw = (int)g.size();
-    ts->dw_tiles = tiles;
-    ts->dw_cls_tiles = ((V + 31) / 32) * ((D + 31) / 32);
-    ts->dw_vec = vec;
+    ts->dw_plan = plan;
     ts->desc_T = T;
     return PTMI_OK;
 }
@@ -1342,7 +1342,7 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     // so every value is the same as in the grouped launch.
     if (tr) {
         SPAN("cls_weight_grad", "bwd", -1);
-        if ((st = launch_gemm_tn_group(ts->dw_desc, 0, 1, ts->dw_cls_tiles, ts->dw_vec, s))) return st;
+        if ((st = launch_gemm_tn_group(ts->dw_desc, 0, 1, ts->dw_plan.first_tiles, ts->dw_plan, s))) return st;
         SPAN_END();
     }
     SPAN_END();
@@ -1400,10 +1400,10 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
     // each layer's dW inside that layer's spans), every RMSNorm dW in one
     if (tr) {
         SPAN("weight_grads", "bwd", -1);
-        if ((st = launch_gemm_tn_group(ts->dw_desc, 1, ts->n_dw, ts->dw_tiles - ts->dw_cls_tiles, ts->dw_vec, s)))
+        if ((st = launch_gemm_tn_group(ts->dw_desc, 1, ts->n_dw, ts->dw_plan.tiles - ts->dw_plan.first_tiles, ts->dw_plan, s)))
             return st;
         SPAN_END();
-    } else if ((st = launch_gemm_tn_group(ts->dw_desc, 0, ts->n_dw, ts->dw_tiles, ts->dw_vec, s))) {
+    } else if ((st = launch_gemm_tn_group(ts->dw_desc, 0, ts->n_dw, ts->dw_plan.tiles, ts->dw_plan, s))) {
         return st;
     }
     SPAN("embedding", "bwd", -1);

@@ -257,3 +257,12 @@ def test_reference_train_step_with_ptmi_matvec_dropin():
         R.ref_ctx_free(cpu)
         R.ref_ctx_free(gpu)
         assert L.ptmi_unregister_weights(P(gpu_blob)) == 0
+
+
+# The grouped weight gradients on 64x64 tiles (K = T-1 past about 600): whole
+# and ragged K, 16-byte and 4-byte rows (odd vocab), widths that are no
+# multiple of a tile.
+@pytest.mark.parametrize("cfg,T", [((128, 260, 1, 4, 4, 4000, 720), 705), ((128, 260, 1, 4, 4, 4001, 660), 642),
+                                   ((184, 400, 1, 2, 2, 3003, 640), 620), ((184, 300, 1, 2, 2, 2004, 704), 704)])
+def test_grouped_weight_gradients_on_large_tiles(cfg, T):
+    check_one_step(cfg, T)
