@@ -53,7 +53,7 @@ def decode_sources_hash(root=ROOT):
 
 # The sources of the training step's kernels (for the in-step kernel times
 # a committed kernel trace measured).
-TRAIN_SOURCES = ["pitorch_amd/csrc/ptmi_train.hip", "pitorch_amd/csrc/ptmi_gemm.hip",
+TRAIN_SOURCES = ["pitorch_amd/csrc/ptmi_train.hip", "pitorch_amd/csrc/ptmi_attention.hip", "pitorch_amd/csrc/ptmi_gemm.hip",
                  "pitorch_amd/csrc/ptmi_internal.h", "pitorch_amd/csrc/ptmi_model.h"]
 
 
