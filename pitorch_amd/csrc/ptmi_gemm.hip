@@ -317,7 +317,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
 
     // One 16x16 block per wave: the 8 MFMAs of a K step go to 8 sums, added
     // pairwise at the end, so each is rounded an eighth as often (64x768x288
-    // and its gradients: 3.0e-7 -> 1.2e-7 from 64-bit sums, 17 us as before).
+    // and its gradients: 3.0e-7 -> 1.2e-7 from 64-bit sums).
     // Not TN: the 32 registers cost the grouped weight gradients occupancy
     // (64 steps of stories15M, T=256: 50.0 -> 52.8 ms).
     constexpr int NC = FM * FN == 1 && !AT ? kChains : 1;
@@ -1142,8 +1142,13 @@ __device__ __forceinline__ int xcd_tile(int b, int total) {
 // index slowest; within a split, neighbouring tiles share the tile of the
 // larger operand (A's rows when M > N, else B's columns).  Smaller grids
 // (at most a few blocks per CU, no reuse to gain) keep the grid's order.
+// The bound of two waves per SIMD keeps the chains (NN and NT) in VGPRs: in
+// AGPRs the register allocator moved all eight of them on every K step
+// (36 moves and 9 waits per two steps; NT 77x496x448 7.45 -> 6.56 us, 6.46 with
+// one chain; 77 NN and NT shapes on these tiles 0.940 -> 0.990 of one chain's
+// speed, the rest is the chains' sum).  TN, with one chain, is level in either.
 template <bool AT, bool BT, int TM, int TN, int P, bool VEC, int EPI = GEMM_EPI_NONE, int NORM = 0>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
+__global__ __launch_bounds__(256, AT ? 1 : 2) void k_gemm(GemmArgs g) {
     const int gx = gridDim.x, gy = gridDim.y, per_z = gx * gy, total = per_z * gridDim.z;
     int m = blockIdx.y, n = blockIdx.x, z = blockIdx.z;
     if (total >= kXcdGrid) {                                        // uniform
@@ -1171,9 +1176,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_dl(GemmArgs g) {
     gemm_tile_dl<AK, BKM, TM, TN, WM, WN>(g, m * TM, n * TN, z);
 }
 
-// The per-layer panel GEMM (grid and tile order as k_gemm).
+// The per-layer panel GEMM (grid, tile order and register bound as k_gemm).
 template <bool BKM, int NSK, int EPI>
-__global__ __launch_bounds__(256) void k_gemm_panel(GemmArgs g) {
+__global__ __launch_bounds__(256, 2) void k_gemm_panel(GemmArgs g) {
     const int gx = gridDim.x, gy = gridDim.y, per_z = gx * gy, total = per_z * gridDim.z;
     int m = blockIdx.y, n = blockIdx.x, z = blockIdx.z;
     if (total >= kXcdGrid) {                                        // uniform
