@@ -800,7 +800,7 @@ struct TileDma {
         }
     }
 };
-constexpr long kMaxSplitLd = 1L << 22;        // 127 rows of it stay below 2^31 bytes
+constexpr long kMaxSplitLd = 1L << 22;        // 128 rows of it take at most 2^31 bytes
 
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -915,6 +915,42 @@ __device__ __forceinline__ void fp32_mma(const GemmArgs &g, int m0, int n0, int 
     static_assert(STAGE <= 4 * T * BK, "one stage");
 }
 
+// A bf16-product tile's output rows: C, or this split's partial product.  Plain
+// sums are added and stored by buffer operations whose elements outside the
+// output have an offset past the descriptor's range: no branch and no 64-bit
+// address per element, and all of a lane's loads of C in flight together (one
+// by one, each load, add and store waited for the one before).  Rows shorter
+// than kMaxSplitLd keep the offsets below 2^31.  TN 32000x768x1024 with
+// accumulate 342 -> 285 us, 17248x669x64 63 -> 31 (47 in 32x32 tiles), NT
+// 1024x8192x64 17.5 -> 15.0 (fp32 128-wide tiles 16.7).
+struct TileOut {
+    __amdgpu_buffer_rsrc_t out, cin;
+    bool add;
+    int ld, rows, cols;                     // rows and columns left from the tile's first
+    __device__ __forceinline__ TileOut(const GemmArgs &g, int m0, int n0, int z) {
+        const bool part = g.partial != nullptr;
+        add = !part && g.accumulate;
+        ld = (int)(part ? g.N : g.ldc);
+        rows = g.M - m0;
+        cols = g.N - n0;
+        const long at = (long)m0 * ld + n0;
+        out = __builtin_amdgcn_make_buffer_rsrc((part ? g.partial + (long)z * g.M * g.N : g.C) + at, (short)0, 0x7fffffff, 0x00020000);
+        cin = __builtin_amdgcn_make_buffer_rsrc((void *)((add ? g.Cin : g.C) + at), (short)0, 0x7fffffff, 0x00020000);
+    }
+    __device__ __forceinline__ int at(int r, int c) const { return r < rows && c < cols ? 4 * (r * ld + c) : kOutside; }
+    // v[i] at offsets off[i]
+    template <int N>
+    __device__ __forceinline__ void put(const float (&v)[N], const int (&off)[N]) const {
+        float c[N];
+        if (add)                                                // uniform
+#pragma unroll
+            for (int i = 0; i < N; i++) c[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(cin, off[i], 0, 0));
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, add ? c[i] + v[i] : v[i]), out, off[i], 0, 0);
+    }
+};
+
 // 128x128 output tile at (m0, n0) over K range split z: 2 x 2 waves of
 // 64x64, K steps of 32 in two LDS stages.  A wave's splits of one 16-k block
 // go between its MFMAs of the block before; the next tile's loads are in
@@ -992,15 +1028,31 @@ __device__ __forceinline__ void gemm_tile_split128(const GemmArgs &g, int m0, in
             for (int v = 0; v < 16; v++) finite = finite && fabsf(acc[f][h][v]) <= 3.4028235e+38f;
     if (__syncthreads_or(!finite)) fp32_mma<AK, BKM, T, E>(g, m0, n0, kb, kend, smem, acc);     // uniform
     // C[(v/4)*8 + 4*(l/32) + v%4][l%32] is component v of lane l
-    const int mb = m0 + wm * 64 + 4 * lh, nb = n0 + wn * 64 + li;
-    const float lrv = g.upd ? *g.lr : 0.0f;
+    const int rb = wm * 64 + 4 * lh, cb = wn * 64 + li;
+    if constexpr (EPI == GEMM_EPI_NONE) {
+        const TileOut o(g, m0, n0, z);
 #pragma unroll
-    for (int f = 0; f < 2; f++)
+        for (int f = 0; f < 2; f++)
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+            for (int h = 0; h < 2; h++) {
+                float s[16];
+                int off[16];
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                store_elem<EPI>(g, acc[f][h][v], mb + f * 32 + (v >> 2) * 8 + (v & 3), nb + h * 32, z, lrv);
+                for (int v = 0; v < 16; v++) {
+                    s[v] = acc[f][h][v];
+                    off[v] = o.at(rb + f * 32 + (v >> 2) * 8 + (v & 3), cb + h * 32);
+                }
+                o.put(s, off);
+            }
+    } else {
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    store_elem<EPI>(g, acc[f][h][v], m0 + rb + f * 32 + (v >> 2) * 8 + (v & 3), n0 + cb + h * 32, z, 0.0f);
+    }
 }
 
 // 64x64 output tile at (m0, n0) over K range split z, K dealt to the four waves:
@@ -1123,6 +1175,14 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < T / NW; e++) sum[e] = red[(e * NW + wave) * T + lane];
+    }
+    if (EPI == GEMM_EPI_NONE && !g.upd) {                       // uniform
+        const TileOut o(g, m0, n0, z);
+        int off[T / NW];
+#pragma unroll
+        for (int e = 0; e < T / NW; e++) off[e] = o.at(e * NW + wave, lane);
+        o.put(sum, off);
+        return;
     }
     const float lrv = g.upd ? *g.lr : 0.0f;
 #pragma unroll
@@ -1287,7 +1347,7 @@ SplitPlan split_plan(int op, int M, int N, int K, size_t ws_floats, int ek) {
 // their partial sums at most as long as the fp32 tiles' would be (the 64
 // tile sums four of its own), so no result is summed in fewer pieces than before.
 struct GemmChoice { int tile, splits, k_per_split; float us, us32; };    // us32: the 32 tiles' estimate
-GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, bool vec, size_t ws_floats, int ek) {
+GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, long ldc, bool vec, size_t ws_floats, int ek) {
     const SplitPlan p = split_plan(op, M, N, K, ws_floats, ek);
     const double mn = (double)M * N, cus = 256.0;
     auto blocks = [&](int T) { return (double)((N + T - 1) / T) * ((M + T - 1) / T); };
@@ -1296,7 +1356,7 @@ GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, bool vec
     const double us32 = 3.2 + reduce(p.splits) +
                         (vec ? 1.0 : 1.5) * steps(p.k_per_split, BK) * (0.1 + 0.19 * std::max(1.0, blocks(32) * p.splits / cus));
     GemmChoice best = {32, p.splits, p.k_per_split, (float)us32, (float)us32};
-    if (lda >= kMaxSplitLd || ldb >= kMaxSplitLd || (ek != GEMM_EPI_NONE && !vec)) return best;
+    if (std::max({lda, ldb, ldc}) >= kMaxSplitLd || (ek != GEMM_EPI_NONE && !vec)) return best;
     // the large short-K weight gradients stay on the 128x96 fp32 tiles
     // (32000x288x64: 22.4 us against 29.4)
     if (op == 1 && vec && ek == GEMM_EPI_NONE && p.splits == 1 && mn >= (4L << 20) && K < 256) return best;
@@ -1331,7 +1391,7 @@ bool gemm_norm_fusable(int M, int N, int K, const float *A, long lda, const floa
     if (M <= 0 || N <= 0 || K <= 0 || K % 4 || lda != K || ldb % 4 || ldb < K) return false;
     if (!A || !B || !al16(A) || !al16(B) || !al16(nm.w) || !al16(nm.xn_out)) return false;
     // the fused norm runs on the 32x32 tiles only, and spares a launch (about 5 us)
-    const GemmChoice ch = gemm_choice(2, M, N, K, lda, ldb, true, 0, epi_kind);
+    const GemmChoice ch = gemm_choice(2, M, N, K, lda, ldb, N, true, 0, epi_kind);
     if (ch.tile != 32 && ch.us + 5.0f < ch.us32) return false;
     if (nm.kind != GEMM_NORM_PLAIN && (!nm.x_out || !al16(nm.x_out))) return false;
     if (nm.kind == GEMM_NORM_SPLITS &&
@@ -1387,7 +1447,7 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
     // 0.769-0.771 ms against 0.778-0.783 with six, and nine and ten were no
     // faster); larger ones take the bf16-product tiles (gemm_choice).  The
     // fused norm runs on the 32x32 tiles.
-    GemmChoice ch = gemm_choice(op, M, N, K, lda, ldb, vec, ws_floats, ek);
+    GemmChoice ch = gemm_choice(op, M, N, K, lda, ldb, ldc, vec, ws_floats, ek);
     if (nk_kind && ch.tile != 32) ch = GemmChoice{32, 1, K, ch.us32, ch.us32};
     const int T = ch.tile;
     const int gx = (N + T - 1) / T, gy = (M + T - 1) / T;
