@@ -145,6 +145,16 @@ int ptmi_matmul_backward_input_batched(float *d_x_all, const float *W,
 int ptmi_gemm_dev(int op, const float *dA, long lda, const float *dB, long ldb,
                   float *dC, long ldc, int M, int N, int K, int accumulate,
                   void *stream);
+/* How ptmi_gemm_dev runs a GEMM of these sizes and row strides: plan[0] x
+ * plan[1] = the output tile of a workgroup, plan[2] = 1 when the products
+ * are fp32 matrix instructions, 0 when each is summed from bf16 parts,
+ * plan[3] = pieces K is cut into.  aligned: both operands start on 16-byte
+ * boundaries and their strides and contiguous extents (K, or M of A^T and N
+ * of B) are multiples of 4.  epilogue: 0 as ptmi_gemm_dev; 1 RoPE and 2 SwiGLU
+ * (op 2), 3 the SwiGLU backward (op 0) as the model's GEMMs fuse them.  Pure host
+ * arithmetic, no device call.  No counterpart in the reference.         */
+int ptmi_gemm_plan(int op, int M, int N, int K, long lda, long ldb, long ldc,
+                   int aligned, int accumulate, int epilogue, int plan[4]);
 /* ptmi_gemm_dev without any allocation.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).

@@ -12,6 +12,7 @@ from ._ffi import (  # noqa: F401
     PtmiError,
     Model,
     decode_step_plan,
+    gemm_plan,
     lib_dir,
     load_host,
     load_ptmi,

@@ -291,12 +291,17 @@ __device__ __forceinline__ void norm_rows_out(const GemmArgs &g, int m0, int j, 
 }
 
 constexpr int kChains = BK / 4;
-// acc[0] = the sum of the 8 partial sums, pairwise
-__device__ __forceinline__ void sum_chains(floatx4 (&acc)[kChains][1][1]) {
+// acc[0] = the sum of the NC partial sums, pairwise
+template <int NC, int FM, int FN>
+__device__ __forceinline__ void sum_chains(floatx4 (&acc)[NC][FM][FN]) {
 #pragma unroll
-    for (int h = kChains / 2; h > 0; h /= 2)
+    for (int h = NC / 2; h > 0; h /= 2)
 #pragma unroll
-        for (int c = 0; c < h; c++) acc[c][0][0] += acc[c + h][0][0];
+        for (int c = 0; c < h; c++)
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) acc[c][i][j] += acc[c + h][i][j];
 }
 
 // One TMxTN output tile of g at (m0, n0) over K range split z.  The LDS
@@ -320,7 +325,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
     // and its gradients: 3.0e-7 -> 1.2e-7 from 64-bit sums).
     // Not TN: the 32 registers cost the grouped weight gradients occupancy
     // (64 steps of stories15M, T=256: 50.0 -> 52.8 ms).
-    constexpr int NC = FM * FN == 1 && !AT ? kChains : 1;
+    // The 64x64 tile's four blocks per wave have four chains each.
+    constexpr int NC = AT ? 1 : FM * FN == 1 ? kChains : 4;
     floatx4 acc[NC][FM][FN];
 #pragma unroll
     for (int c = 0; c < NC; c++)
@@ -1331,54 +1337,71 @@ SplitPlan split_plan(int op, int M, int N, int K, size_t ws_floats, int ek) {
     return SplitPlan{chosen, (K + kps - 1) / kps, kps};
 }
 
-// Tile and K split of a GEMM: 32 (fp32 MFMA tiles, `splits` from split_plan),
-// 64 or 128 (bf16 products).  The smallest estimate of the launch's time in
-// µs, fitted to launches back to back on the MI355X (256 CUs; n = blocks per
-// CU, measured -> estimated):
-//   32:  3.2 + steps * (0.1 + 0.19 n), n >= 1, steps of 32 k:
-//        256x512x1536 17.3 -> 17.1, 1024x768x768 17.8 -> 19.3, 1024x2048x768 40 -> 42
-//   64:  4 + ceil(n) * (2.6 + 0.65 * blocks of 64 k):
-//        256x768x768 12.7 -> 14.4, 1024x2048x768 25.5 -> 24.8, 1024x4096x768 45.9 -> 45.6
-//   128: 5 + ceil(n) * (1.5 + 1.42 * steps), n >= 1.5:
-//        256x32000x288 36 -> 34, 1024x32000x768 277 -> 290
+// Kernel and K split of a GEMM.  GEMM_32: 32x32 fp32 MFMA tiles, K split by
+// split_plan; GEMM_64 and GEMM_128: bf16 products, the smaller estimate of a launch's
+// time in us, fitted to 1850 launches back to back on the MI355X (256 CUs;
+// n = blocks per CU; measured -> estimated; over those the choice takes 0.4%
+// longer than the fastest of the three would):
+//   GEMM_32:  3.2 + i * (n - 1) + steps * (0.1 + s * n), n >= 1, steps of 32 k; i, s =
+//        0.4, 0.18 NT, 0.3, 0.19 NN, 0.2, 0.19 TN: NT 827x1600x376 16.9 -> 16.9,
+//        NN 1024x4096x64 13.7 -> 14.0, TN 1184x2000x176 15.1 -> 15.7, 36x160x6725 10.1 -> 10.3
+//   GEMM_64:  3.6 + ceil(n) * (1.85 + 0.65 * steps), at least two steps of 64 k:
+//        131x960x896 10.8 -> 11.3 (split), 1024x2048x768 25.1 -> 22.9, 423x3808x1408 34.5 -> 35.9
+//   GEMM_128: 3.2 + ceil(n) * (2.8 + 1.3 * steps), n >= 1, steps of 32 k, 2.0 each at
+//        n = 1 (a lone block per CU): 1024x8192x64 15.0 -> 14.0, 1024x32000x768 265 -> 275,
+//        1024x4096x96 12.3 -> 12.0
 //   split K: + 3 and the partials' traffic at 3.5 TB/s.
 // Without 16-byte rows the 32 tiles' loads cost 1.5x per step, the others' 1.2x
-// (501x517x1003: 24.8 against 16.9 µs with three splits).  The bf16 tiles keep
+// (501x517x1003: 24.6 against 16.1 us with three splits).  The bf16 tiles keep
 // their partial sums at most as long as the fp32 tiles' would be (the 64
-// tile sums four of its own), so no result is summed in fewer pieces than before.
-struct GemmChoice { int tile, splits, k_per_split; float us, us32; };    // us32: the 32 tiles' estimate
-GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, long ldc, bool vec, size_t ws_floats, int ek) {
+// tile sums four of its own), so no result is summed in fewer pieces.
+// Two fp32 tiles stay where they are faster than all three:
+//   GEMM_DL (128x96, direct to LDS): TN outputs of 4 Mi elements and more, one
+//        K step and no accumulate: 32000x288x16 14.4 us against 15.6 (GEMM_128); with
+//        accumulate 4096x1100x16 16.8 against 11.5, at K = 48 20.6 against 19.4.
+//   GEMM_64F (64x64): NT outputs of that size from at most 64 rows, which leave half
+//        of a 128 tile empty, K <= 96: 64x65600x20 10.3 against 13.9 (14.2, GEMM_32),
+//        at K = 96 16.9 against 18.0, at K = 128 19.4 against 19.3 (GEMM_64).
+enum GemmKind { GEMM_32, GEMM_64F, GEMM_DL, GEMM_64, GEMM_128 };
+struct GemmChoice {
+    GemmKind kind;
+    int tm, tn, splits, k_per_split;
+    float us, us32;                                             // its estimate and the 32 tiles'
+};
+GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, long ldc, bool vec, bool accumulate,
+                       size_t ws_floats, int ek) {
     const SplitPlan p = split_plan(op, M, N, K, ws_floats, ek);
     const double mn = (double)M * N, cus = 256.0;
     auto blocks = [&](int T) { return (double)((N + T - 1) / T) * ((M + T - 1) / T); };
     auto reduce = [&](int s) { return s > 1 ? 3.0 + (s + 1) * mn * 4.0 / 3.5e6 : 0.0; };
     auto steps = [&](int k, int per) { return (double)((k + per - 1) / per); };
-    const double us32 = 3.2 + reduce(p.splits) +
-                        (vec ? 1.0 : 1.5) * steps(p.k_per_split, BK) * (0.1 + 0.19 * std::max(1.0, blocks(32) * p.splits / cus));
-    GemmChoice best = {32, p.splits, p.k_per_split, (float)us32, (float)us32};
-    if (std::max({lda, ldb, ldc}) >= kMaxSplitLd || (ek != GEMM_EPI_NONE && !vec)) return best;
-    // the large short-K weight gradients stay on the 128x96 fp32 tiles
-    // (32000x288x64: 22.4 us against 29.4)
-    if (op == 1 && vec && ek == GEMM_EPI_NONE && p.splits == 1 && mn >= (4L << 20) && K < 256) return best;
-    // long K and large NT outputs always leave the 32x32 tiles
-    const bool leave = K >= 4096 || (op == 2 && mn >= (4L << 20));
-    if (!leave && us32 < 7.0) return best;                       // below any of the others
-    if (leave) best.us = 1e30f;
+    const double fill[3] = {0.3, 0.2, 0.4}, per_step[3] = {0.19, 0.19, 0.18};
+    const double n32 = std::max(1.0, blocks(32) * p.splits / cus);
+    const double us32 = 3.2 + fill[op] * (n32 - 1) + reduce(p.splits) +
+                        (vec ? 1.0 : 1.5) * steps(p.k_per_split, BK) * (0.1 + per_step[op] * n32);
+    GemmChoice best = {GEMM_32, 32, 32, p.splits, p.k_per_split, (float)us32, (float)us32};
+    const bool large = mn >= (4L << 20), split_ok = std::max({lda, ldb, ldc}) < kMaxSplitLd;
+    if (ek == GEMM_EPI_NONE && op == 1 && vec && p.splits == 1 && large && (!split_ok || (K < 48 && !accumulate)))
+        return GemmChoice{GEMM_DL, 128, 96, 1, K, (float)us32, (float)us32};
+    if (ek == GEMM_EPI_NONE && op == 2 && large && M <= 64 && K <= 96)
+        return GemmChoice{GEMM_64F, 64, 64, 1, K, (float)us32, (float)us32};
+    if (!split_ok || (ek != GEMM_EPI_NONE && !vec)) return best;
+    if (us32 < 7.0) return best;                                 // below any of the others
     const int max_s = ek != GEMM_EPI_NONE ? 1 : std::max(1, std::min(64, K / 128));
     for (int s = 1; s <= max_s; s += 1 + s / 8) {
         const double red = reduce(s);
-        if (s > 1 && ((size_t)s * M * N > std::min(ws_floats, kScratchFloats) || 7.0 + red > best.us)) break;
+        if (s > 1 && ((size_t)s * M * N > std::min(ws_floats, kScratchFloats) || 6.7 + red > best.us)) break;
         const int kps = ((K + s - 1) / s + BK - 1) / BK * BK, splits = (K + kps - 1) / kps;
         for (int T = 64; T <= 128; T += 64) {
             if (kps > (T == 64 ? 4 : 1) * p.k_per_split) continue;
             const double n = blocks(T) * splits / cus;
-            if (T == 128 && n < 1.5) continue;
-            const double per = T == 64 ? 2.6 + 0.65 * steps(kps, 64) : 1.5 + 1.42 * steps(kps, BK);
-            const double us = (T == 64 ? 4.0 : 5.0) + (vec ? 1.0 : 1.2) * std::ceil(n) * per + red;
-            if (us < best.us) best = GemmChoice{T, splits, splits > 1 ? kps : K, (float)us, (float)us32};
+            if (T == 128 && n < 1.0) continue;
+            const double per = T == 64 ? 1.85 + 0.65 * std::max(2.0, steps(kps, 64)) : 2.8 + (n > 1.0 ? 1.3 : 2.0) * steps(kps, BK);
+            const double us = (T == 64 ? 3.6 : 3.2) + (vec ? 1.0 : 1.2) * std::ceil(n) * per + red;
+            if (us < best.us)
+                best = GemmChoice{T == 64 ? GEMM_64 : GEMM_128, T, T, splits, splits > 1 ? kps : K, (float)us, (float)us32};
         }
     }
-    if (best.tile == 32) best.us = (float)us32;
     return best;
 }
 
@@ -1391,8 +1414,8 @@ bool gemm_norm_fusable(int M, int N, int K, const float *A, long lda, const floa
     if (M <= 0 || N <= 0 || K <= 0 || K % 4 || lda != K || ldb % 4 || ldb < K) return false;
     if (!A || !B || !al16(A) || !al16(B) || !al16(nm.w) || !al16(nm.xn_out)) return false;
     // the fused norm runs on the 32x32 tiles only, and spares a launch (about 5 us)
-    const GemmChoice ch = gemm_choice(2, M, N, K, lda, ldb, N, true, 0, epi_kind);
-    if (ch.tile != 32 && ch.us + 5.0f < ch.us32) return false;
+    const GemmChoice ch = gemm_choice(2, M, N, K, lda, ldb, N, true, false, 0, epi_kind);
+    if (ch.kind != GEMM_32 && ch.us + 5.0f < ch.us32) return false;
     if (nm.kind != GEMM_NORM_PLAIN && (!nm.x_out || !al16(nm.x_out))) return false;
     if (nm.kind == GEMM_NORM_SPLITS &&
         (nm.pk.splits < 1 || nm.pk.splits > kNormSplits || !nm.pk.parts || !al16(nm.pk.parts) || nm.pk.stride % 4 ||
@@ -1447,10 +1470,9 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
     // 0.769-0.771 ms against 0.778-0.783 with six, and nine and ten were no
     // faster); larger ones take the bf16-product tiles (gemm_choice).  The
     // fused norm runs on the 32x32 tiles.
-    GemmChoice ch = gemm_choice(op, M, N, K, lda, ldb, ldc, vec, ws_floats, ek);
-    if (nk_kind && ch.tile != 32) ch = GemmChoice{32, 1, K, ch.us32, ch.us32};
-    const int T = ch.tile;
-    const int gx = (N + T - 1) / T, gy = (M + T - 1) / T;
+    GemmChoice ch = gemm_choice(op, M, N, K, lda, ldb, ldc, vec, accumulate, ws_floats, ek);
+    if (nk_kind && ch.kind != GEMM_32) ch = GemmChoice{GEMM_32, 32, 32, 1, K, ch.us32, ch.us32};
+    const int gx = (N + ch.tn - 1) / ch.tn, gy = (M + ch.tm - 1) / ch.tm;
     const int splits = ch.splits;
     g.k_per_split = ch.k_per_split;
     g.partial = splits > 1 ? ws : nullptr;
@@ -1484,8 +1506,8 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
         if (!vec || splits != 1) return set_error(PTMI_ERR_STATE, "gemm: fused norm without whole-K float4 tiles");
         fn = fused_norm[ek == GEMM_EPI_SWIGLU][nk_kind - 1];
     }
-    int threads = 256;
-    if (T != 32) {
+    const bool split = ch.kind == GEMM_64 || ch.kind == GEMM_128;
+    if (split) {
 #define PTMI_SPLIT_KERNELS(T_)                                                                                        \
     {{k_gemm_split<false, true, T_, 1, 0>, k_gemm_split<true, true, T_, 1, 0>, k_gemm_split<false, false, T_, 1, 0>}, \
      {k_gemm_split<false, true, T_, 4, 0>, k_gemm_split<true, true, T_, 4, 0>, k_gemm_split<false, false, T_, 4, 0>}}
@@ -1496,7 +1518,8 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
              k_gemm_split<false, true, 64, 4, GEMM_EPI_SWIGLU_BWD>},
             {k_gemm_split<false, false, 128, 4, GEMM_EPI_ROPE>, k_gemm_split<false, false, 128, 4, GEMM_EPI_SWIGLU>,
              k_gemm_split<false, true, 128, 4, GEMM_EPI_SWIGLU_BWD>}};
-        fn = ek != GEMM_EPI_NONE ? fused[T == 128][ek - 1] : plain[T == 128][vec][op];
+        const int big = ch.kind == GEMM_128;
+        fn = ek != GEMM_EPI_NONE ? fused[big][ek - 1] : plain[big][vec][op];
     }
     // Per-layer 32x32 GEMMs with at most 9 K tiles per split: the panel
     // kernel, every K tile in flight at once.  PTMI_GEMM_PANEL is a bit mask
@@ -1509,7 +1532,7 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
     static const int use_panel = [] { const char *e = getenv("PTMI_GEMM_PANEL"); return e ? atoi(e) & 7 : 3; }();
     const int nk_split = (ch.k_per_split + BK - 1) / BK;
     const int panel_bit = op == 2 ? 1 : ek == GEMM_EPI_SWIGLU_BWD ? 2 : 4;
-    if ((use_panel & panel_bit) && T == 32 && vec && !nk_kind && op != 1 && nk_split <= 9) {
+    if ((use_panel & panel_bit) && ch.kind == GEMM_32 && vec && !nk_kind && op != 1 && nk_split <= 9) {
         using PFn = void (*)(GemmArgs);
         static const PFn panel[2][2][4] = {
             {{k_gemm_panel<false, 6, GEMM_EPI_NONE>, k_gemm_panel<false, 6, GEMM_EPI_ROPE>,
@@ -1522,14 +1545,9 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
         const PFn pf = panel[op == 0][nk_split > 6][ei];
         if (pf) fn = pf;
     }
-    // The large short-K weight gradients (the classifier's at T <= 256) take
-    // the direct-to-LDS tiles.
-    if (T == 32 && vec && ek == GEMM_EPI_NONE && splits == 1 && op == 1 && (long)M * N >= (4L << 20)) {
-        grid = dim3((unsigned)((N + 95) / 96), (unsigned)((M + 127) / 128), 1);
-        fn = k_gemm_dl<true, true, 128, 96, 4, 2>;
-        threads = 512;
-    }
-    hipLaunchKernelGGL(fn, grid, dim3(threads), 0, s, g);
+    if (ch.kind == GEMM_64F) fn = vec ? k_gemm<false, true, 64, 64, kRing32, true> : k_gemm<false, true, 64, 64, kRing32, false>;
+    if (ch.kind == GEMM_DL) fn = k_gemm_dl<true, true, 128, 96, 4, 2>;
+    hipLaunchKernelGGL(fn, grid, dim3(ch.kind == GEMM_DL ? 512 : 256), 0, s, g);
     PTMI_HIP(hipGetLastError());
     if (splits > 1 && defer) {
         *defer = SplitK{ws, splits, (long)M * N};
@@ -1693,6 +1711,18 @@ int ptmi_gemm_dev(int op, const float *dA, long lda, const float *dB, long ldb, 
     if (!ws) return ptmi_last_status();
     return launch_gemm(op, dA, lda, dB, ldb, dC, ldc, M, N, K, accumulate, ws, ws_n,
                        stream ? (hipStream_t)stream : lib_stream());
+}
+
+int ptmi_gemm_plan(int op, int M, int N, int K, long lda, long ldb, long ldc, int aligned, int accumulate, int epilogue,
+                   int plan[4]) {
+    if (!plan || op < 0 || op > 2 || M <= 0 || N <= 0 || K <= 0 || epilogue < GEMM_EPI_NONE || epilogue > GEMM_EPI_SWIGLU_BWD)
+        return set_error(PTMI_ERR_ARG, "ptmi_gemm_plan: bad arguments");
+    const GemmChoice c = gemm_choice(op, M, N, K, lda, ldb, ldc, aligned != 0, accumulate != 0, gemm_dev_ws_floats(M, N), epilogue);
+    plan[0] = c.tm;
+    plan[1] = c.tn;
+    plan[2] = c.kind != GEMM_64 && c.kind != GEMM_128;
+    plan[3] = c.splits;
+    return PTMI_OK;
 }
 
 int ptmi_sgemm_rect(const float *A, const float *B, float *C, int M, int K, int N, int accumulate) {

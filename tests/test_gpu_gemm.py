@@ -308,6 +308,32 @@ def test_gemm_dev_split_tiles_non_finite(op, M, N, K, acc, pad):
     assert bound_ok(got[clean], a @ b, np.abs(a) @ np.abs(b), K)
 
 
+# Large outputs of short K on each of the kernels that take them (as
+# tests/test_gemm_plan.py pins the choice), ragged in every size; C's padding
+# columns are NaN before and after.
+@pytest.mark.parametrize("op,M,N,K,acc,pad,kernel", [
+    (2, 64, 65600, 1, 0, 0, (64, 64, 1)), (2, 63, 66601, 7, 1, 3, (64, 64, 1)), (2, 33, 131100, 96, 0, 4, (64, 64, 1)),
+    (2, 300, 20001, 7, 1, 1, (128, 128, 0)), (2, 1024, 8192, 16, 0, 4, (128, 128, 0)), (0, 1023, 8191, 17, 1, 2, (128, 128, 0)),
+    (1, 17247, 669, 41, 1, 3, (128, 128, 0)), (1, 32000, 132, 33, 1, 4, (128, 128, 0)), (1, 32004, 132, 31, 0, 4, (128, 96, 1)),
+])
+def test_gemm_dev_short_k(op, M, N, K, acc, pad, kernel):
+    assert pa.gemm_plan(op, M, N, K, pad=pad, accumulate=acc)[:3] == kernel
+    A, B = ints((M, K), 51), ints((K, N), 52)
+    C0 = ints((M, N), 53) if acc else np.full((M, N), np.nan, np.float32)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    c = np.pad(C0, ((0, 0), (0, pad)), constant_values=np.nan)
+    stored = [np.ascontiguousarray(np.pad(x, ((0, 0), (0, pad)), constant_values=np.nan))
+              for x in (A.T if op == 1 else A, B.T if op == 2 else B)]
+    dA, dB, dC = (DeviceArray.from_host(x) for x in (*stored, c))
+    L = pa.load_ptmi()
+    assert L.ptmi_gemm_dev(op, dA.ptr, stored[0].shape[1], dB.ptr, stored[1].shape[1], dC.ptr, N + pad, M, N, K, acc, None) == 0
+    assert L.ptmi_sync() == 0
+    got = dC.download().reshape(M, N + pad)
+    assert np.array_equal(got[:, :N], (ref + C0 if acc else ref).astype(np.float32)) and np.all(np.isnan(got[:, N:]))
+    for d in (dA, dB, dC):
+        d.free()
+
+
 def test_gemm_errors():
     L = pa.load_ptmi()
     A = np.ones((4, 4), np.float32)
