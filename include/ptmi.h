@@ -141,7 +141,11 @@ int ptmi_matmul_backward_input_batched(float *d_x_all, const float *W,
 /* Device-pointer forms.  op: 0 = NN  C(+)=A.B,      A[M,K]  B[K,N]
  *                            1 = TN  C(+)=A^T.B,    A[K,M]  B[K,N]
  *                            2 = NT  C(+)=A.B^T,    A[M,K]  B[N,K]
- * lda/ldb/ldc are row strides in floats.                                */
+ * lda/ldb/ldc are row strides in floats.  Every sum is held to the bound of
+ * K fp32 roundings, K*2^-24*sum|a*b|, also where the operands, products or
+ * sums are subnormal, infinite or NaN.  Middle and large products with
+ * K >= 16 are summed from bf16 parts in fp32 (ptmi_gemm_plan tells which):
+ * there a lone product among zeros may be 3*2^-24 off instead of 2^-24.  */
 int ptmi_gemm_dev(int op, const float *dA, long lda, const float *dB, long ldb,
                   float *dC, long ldc, int M, int N, int K, int accumulate,
                   void *stream);

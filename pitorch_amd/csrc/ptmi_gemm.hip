@@ -718,20 +718,24 @@ __device__ __forceinline__ void gemm_tile_panel(const GemmArgs &g, int m0, int n
 // ── fp32 products on the bf16 matrix cores ───────────────────────────────
 // The large and middle GEMMs.  v_mfma_f32_32x32x16_bf16 runs 16x the
 // multiply-adds per cycle of v_mfma_f32_32x32x2_f32, and an fp32 number is
-// exactly the sum of three bf16: x = h + m + l, h the nearest bf16, m the top
-// 8 bits of x - h, l the rest (24 significant bits in all).  a*b is taken as
+// exactly the sum of three bf16: x = h + m + l, h the nearest bf16, m the
+// nearest to x - h, l the rest (24 significant bits in all).  a*b is taken as
 // the six largest of the nine partial products, smallest first into one fp32
-// accumulator: al*bh, ah*bl, am*bm, am*bh, ah*bm, ah*bh.  The three dropped are below
-// 2^-24 of |a*b| and of either sign (h is rounded, not cut), and the
-// accumulator rounds 6 times per 16 k instead of 16 times, so results are
-// nearer to 64-bit sums than the fp32 MFMA tiles' (relative error at K = 768
+// accumulator: al*bh, ah*bl, am*bm, am*bh, ah*bm, ah*bh.  The three dropped are
+// together below 2^-24 of |a*b| (+ 2^-33) and of either sign (h and m are rounded,
+// not cut), and the accumulator rounds 6 times per 16 k instead of 16 times, so
+// results are nearer to 64-bit sums than the fp32 MFMA tiles' (relative error at K = 768
 // and 2048: 5.0e-7 and 8.1e-7 before, 4.2e-7 and 6.9e-7 in 128x128 tiles,
 // 2.1e-7 and 3.4e-7 in 64x64 tiles, whose four waves each sum a quarter of
-// K).  Numbers below 2^-109 lose low bits (bf16 reaches down to 2^-133).  A
-// tile with a non-finite sum is computed again with fp32 MFMAs, so
-// infinities, NaNs and numbers that round past the bf16 range come out as
-// the fp32 tiles give them.
-// What bounds it: the MFMAs (32 cycles each) and the splits (7 VALU
+// K).  A single product among zeros is up to 3 x 2^-24 off, where fp32 MFMAs
+// round it to nearest (2^-24): sums of fewer than 16 terms are left to them.
+// A tile is computed again with fp32 MFMAs, and so comes out as the fp32 tiles
+// give it, where a sum is not finite (infinities, NaNs, numbers that round past
+// the bf16 range) or subnormal, or where an operand has bits below bf16's
+// smallest number, 2^-133, as operands below 2^-109 can.  Rounding m and
+// watching for such bits cost about 1.5% in 64x64 tiles and 0 to 6% in 128x128 ones
+// (NT 1024x32000x768 271 -> 289 us).
+// What bounds it: the MFMAs (32 cycles each) and the splits (8 VALU
 // instructions per MFMA) issue side by side; with the splits taken out the same
 // kernels reach 180-195 TFLOP/s, the bf16 matrix rate under the card's power limit.
 //
@@ -806,6 +810,7 @@ struct TileDma {
         }
     }
 };
+constexpr int kShortK = 16;                   // fewer terms are left to fp32 MFMAs
 constexpr long kMaxSplitLd = 1L << 22;        // 128 rows of it take at most 2^31 bytes
 
 typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -813,19 +818,22 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
-// x[e] = o[0][e] + o[1][e] + o[2][e] (see above).
-__device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&o)[3]) {
+// x[e] = o[0][e] + o[1][e] + o[2][e] (see above).  h and m are rounded to nearest, so
+// |m| <= 2^-8 and |l| <= 2^-17 of x's leading power of two (m cut instead: 2^-16).  The
+// low halves of `lost` collect what l's bf16 cannot hold (x below 2^-109).
+__device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&o)[3], unsigned &lost) {
     constexpr unsigned kTop = 0xffff0000u, kHighHalves = 0x07060302u;
     uintx4 h, m, l;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const floatx2 v = {x[2 * e], x[2 * e + 1]};
         h[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
-        const float r0 = v.x - __uint_as_float(h[e] << 16), r1 = v.y - __uint_as_float(h[e] & kTop);
-        const unsigned u0 = __float_as_uint(r0), u1 = __float_as_uint(r1);
-        const float l0 = r0 - __uint_as_float(u0 & kTop), l1 = r1 - __uint_as_float(u1 & kTop);
-        m[e] = __builtin_amdgcn_perm(u1, u0, kHighHalves);
-        l[e] = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), kHighHalves);
+        const floatx2 r = {v.x - __uint_as_float(h[e] << 16), v.y - __uint_as_float(h[e] & kTop)};
+        m[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+        const unsigned l0 = __float_as_uint(r.x - __uint_as_float(m[e] << 16)), l1 = __float_as_uint(r.y - __uint_as_float(m[e] & kTop));
+        l[e] = __builtin_amdgcn_perm(l1, l0, kHighHalves);
+        lost |= l0 | l1;
+        asm("" : "+v"(lost));                                   // now: gathered later, the l would be held till then
     }
     o[0] = __builtin_bit_cast(bf16x8, h);
     o[1] = __builtin_bit_cast(bf16x8, m);
@@ -836,11 +844,11 @@ __device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8 (&o)[3]) 
 struct RawFrags { float a[2][8], b[2][8]; };
 struct SplitFrags { bf16x8 a[2][3], b[2][3]; };
 
-__device__ __forceinline__ void split_frags(const RawFrags &x, SplitFrags &o) {
+__device__ __forceinline__ void split_frags(const RawFrags &x, SplitFrags &o, unsigned &lost) {
 #pragma unroll
-    for (int f = 0; f < 2; f++) split_bf16(x.a[f], o.a[f]);
+    for (int f = 0; f < 2; f++) split_bf16(x.a[f], o.a[f], lost);
 #pragma unroll
-    for (int f = 0; f < 2; f++) split_bf16(x.b[f], o.b[f]);
+    for (int f = 0; f < 2; f++) split_bf16(x.b[f], o.b[f], lost);
 }
 
 __device__ __forceinline__ void split_products(const SplitFrags &x, floatx16 (&acc)[2][2]) {
@@ -852,6 +860,12 @@ __device__ __forceinline__ void split_products(const SplitFrags &x, floatx16 (&a
 #pragma unroll
             for (int h = 0; h < 2; h++)
                 acc[f][h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.a[f][pa[p]], x.b[h][pb[p]], acc[f][h], 0, 0, 0);
+}
+
+// A sum the bf16 products do not vouch for: not finite, or subnormal (its
+// products' parts are below what fp32 sums hold).
+__device__ __forceinline__ bool unsure(float s) {
+    return __builtin_amdgcn_classf(s, 0x297);                   // NaN, infinity, subnormal
 }
 
 template <int F>
@@ -882,7 +896,8 @@ __device__ __forceinline__ void block_loads_and_reads() {
 }
 
 // The T x T tile at (m0, n0) over k in [kb, kend) with fp32 MFMAs, on 2 x 2
-// waves of T/2 x T/2: the non-finite case above.  smem: 4*T*BK floats.
+// waves of T/2 x T/2: the cases above that bf16 products do not cover.  smem:
+// 4*T*BK floats.
 template <bool AK, bool BKM, int T, int E>
 __device__ __forceinline__ void fp32_mma(const GemmArgs &g, int m0, int n0, int kb, int kend, float *smem,
                                          floatx16 (&acc)[T / 64][T / 64]) {
@@ -900,8 +915,7 @@ __device__ __forceinline__ void fp32_mma(const GemmArgs &g, int m0, int n0, int 
         da.issue(g.A + (AK ? (long)k0 * g.lda + m0 : (long)m0 * g.lda + k0), 0x7fffffff, smem, wave);
         db.issue(g.B + (BKM ? (long)k0 * g.ldb + n0 : (long)n0 * g.ldb + k0), 0x7fffffff, smem + T * BK, wave);
         block_loads_and_reads();
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
+        for (int q = 0; q < 2 && k0 + 16 * q < kend; q++) {     // uniform
             float xa[F][8], xb[F][8];
 #pragma unroll
             for (int f = 0; f < F; f++) {
@@ -998,19 +1012,20 @@ __device__ __forceinline__ void gemm_tile_split128(const GemmArgs &g, int m0, in
     };
     floatx16 acc[2][2];
     zero_acc<2>(acc);
-    if (nk > 0) {                                               // uniform
+    unsigned lost = 0;
+    if (nk > 0 && g.K >= kShortK) {                             // uniform
         SplitFrags s0, s1;
         place(min(BK, kend - kb));
         issue(0);
         block_loads_and_reads();
         if (nk > 1) issue(1);
         read(0, 0);
-        split_frags(x, s0);
+        split_frags(x, s0, lost);
         for (int s = 0; s < nk; s++) {
             read(s, 1);
             __builtin_amdgcn_sched_barrier(0);
             split_products(s0, acc);
-            split_frags(x, s1);
+            split_frags(x, s1, lost);
             __builtin_amdgcn_sched_barrier(0);
             if (s + 1 < nk) {
                 // tile s+1 is in, and every wave has read tile s, whose
@@ -1021,18 +1036,18 @@ __device__ __forceinline__ void gemm_tile_split128(const GemmArgs &g, int m0, in
             }
             __builtin_amdgcn_sched_barrier(0);
             split_products(s1, acc);
-            split_frags(x, s0);
+            split_frags(x, s0, lost);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    bool finite = true;
+    bool again = g.K < kShortK || (lost & 0xffffu) != 0;
 #pragma unroll
     for (int f = 0; f < 2; f++)
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) finite = finite && fabsf(acc[f][h][v]) <= 3.4028235e+38f;
-    if (__syncthreads_or(!finite)) fp32_mma<AK, BKM, T, E>(g, m0, n0, kb, kend, smem, acc);     // uniform
+            for (int v = 0; v < 16; v++) again |= unsure(acc[f][h][v]);
+    if (__syncthreads_or(again)) fp32_mma<AK, BKM, T, E>(g, m0, n0, kb, kend, smem, acc);     // uniform
     // C[(v/4)*8 + 4*(l/32) + v%4][l%32] is component v of lane l
     const int rb = wm * 64 + 4 * lh, cb = wn * 64 + li;
     if constexpr (EPI == GEMM_EPI_NONE) {
@@ -1116,7 +1131,8 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
     };
     floatx16 acc[2][2];
     zero_acc<2>(acc);
-    if (n > 0) {                                                // wave-uniform
+    unsigned lost = 0;
+    if (n > 0 && g.K >= kShortK) {                              // wave-uniform
         SplitFrags s0, s1;
         if (first) place(tail);
         else place(KD);
@@ -1126,7 +1142,7 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
         wait_vmcnt<LPT>();
         asm volatile("" ::: "memory");
         read(0);
-        split_frags(x, s0);
+        split_frags(x, s0, lost);
         wait_reads();
         issue(2, 0);
         for (int j = 0; j < n; j += 2) {
@@ -1136,7 +1152,7 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
             read(1);
             __builtin_amdgcn_sched_barrier(0);
             split_products(s0, acc);
-            split_frags(x, s1);
+            split_frags(x, s1, lost);
             __builtin_amdgcn_sched_barrier(0);
             wait_reads();
             issue(j + 3, 1);
@@ -1145,7 +1161,7 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
             read(0);
             __builtin_amdgcn_sched_barrier(0);
             split_products(s1, acc);
-            split_frags(x, s0);
+            split_frags(x, s0, lost);
             __builtin_amdgcn_sched_barrier(0);
             wait_reads();
             issue(j + 4, 0);
@@ -1165,14 +1181,14 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
     __syncthreads();
     // wave w sums rows w, w+4, ...; lane = column
     float sum[T / NW];
-    bool finite = true;
+    bool again = g.K < kShortK || (lost & 0xffffu) != 0;
 #pragma unroll
     for (int e = 0; e < T / NW; e++) {
         const float *p = red + (e * NW + wave) * T + (lane ^ ((e & 1) << 5));      // row bit 2 = bit 0 of e
         sum[e] = ((p[0] + p[T * T]) + p[2 * T * T]) + p[3 * T * T];
-        finite = finite && fabsf(sum[e]) <= 3.4028235e+38f;
+        again |= unsure(sum[e]);
     }
-    if (__syncthreads_or(!finite)) {                            // uniform
+    if (__syncthreads_or(again)) {                            // uniform
         floatx16 fa[1][1];
         fp32_mma<AK, BKM, T, E>(g, m0, n0, kb, kend, smem, fa);
 #pragma unroll
