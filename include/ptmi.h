@@ -145,7 +145,12 @@ int ptmi_matmul_backward_input_batched(float *d_x_all, const float *W,
  * K fp32 roundings, K*2^-24*sum|a*b|, also where the operands, products or
  * sums are subnormal, infinite or NaN.  Middle and large products with
  * K >= 16 are summed from bf16 parts in fp32 (ptmi_gemm_plan tells which):
- * there a lone product among zeros may be 3*2^-24 off instead of 2^-24.  */
+ * there a lone product among zeros may be 3*2^-24 off instead of 2^-24.
+ * A GEMM whose K is cut (ptmi_gemm_plan: plan[3] > 1) adds its pieces up in a
+ * workspace that all calls on streams other than the library's share: two such
+ * calls that can overlap race.  On those streams only long K into few output
+ * tiles is cut (32x32 tiles: fewer than 128, K > 288; K >= 4096: fewer than
+ * 512 of 64x64); other GEMMs share nothing.                             */
 int ptmi_gemm_dev(int op, const float *dA, long lda, const float *dB, long ldb,
                   float *dC, long ldc, int M, int N, int K, int accumulate,
                   void *stream);
@@ -155,10 +160,11 @@ int ptmi_gemm_dev(int op, const float *dA, long lda, const float *dB, long ldb,
  * plan[3] = pieces K is cut into.  aligned: both operands start on 16-byte
  * boundaries and their strides and contiguous extents (K, or M of A^T and N
  * of B) are multiples of 4.  epilogue: 0 as ptmi_gemm_dev; 1 RoPE and 2 SwiGLU
- * (op 2), 3 the SwiGLU backward (op 0) as the model's GEMMs fuse them.  Pure host
+ * (op 2), 3 the SwiGLU backward (op 0) as the model's GEMMs fuse them.
+ * callers_stream: 1 for a call on a stream other than the library's.  Pure host
  * arithmetic, no device call.  No counterpart in the reference.         */
 int ptmi_gemm_plan(int op, int M, int N, int K, long lda, long ldb, long ldc,
-                   int aligned, int accumulate, int epilogue, int plan[4]);
+                   int aligned, int accumulate, int epilogue, int callers_stream, int plan[4]);
 /* ptmi_gemm_dev without any allocation.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).

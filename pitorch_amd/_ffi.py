@@ -72,7 +72,7 @@ def load_ptmi():
                                  i, i, i, i, _vp])
     _sig(L, "ptmi_gemm_dev_noalloc", i, [i, _vp, ctypes.c_long, _vp, ctypes.c_long, _vp, ctypes.c_long,
                                          i, i, i, i, _vp])
-    _sig(L, "ptmi_gemm_plan", i, [i, i, i, i, ctypes.c_long, ctypes.c_long, ctypes.c_long, i, i, i, _c_int_p])
+    _sig(L, "ptmi_gemm_plan", i, [i, i, i, i, ctypes.c_long, ctypes.c_long, ctypes.c_long, i, i, i, i, _c_int_p])
     _sig(L, "ptmi_model_create", i, [_vp, sz, i, ctypes.POINTER(_vp)])
     _sig(L, "ptmi_model_destroy", None, [_vp])
     _sig(L, "ptmi_model_config", i, [_vp, _c_int_p])
@@ -165,7 +165,7 @@ def decode_step_plan(cfg, cus, per_cu):
     return reason.value, grid.value, units.value
 
 
-def gemm_plan(op, M, N, K, pad=0, aligned=None, accumulate=0, epilogue=0):
+def gemm_plan(op, M, N, K, pad=0, aligned=None, accumulate=0, epilogue=0, callers_stream=0):
     """ptmi_gemm_plan of dense operands with `pad` floats after each row:
     (tile rows, tile columns, fp32 products, splits).  aligned: by default
     whether the strides and contiguous extents are multiples of 4."""
@@ -174,7 +174,8 @@ def gemm_plan(op, M, N, K, pad=0, aligned=None, accumulate=0, epilogue=0):
     if aligned is None:
         aligned = not any(v % 4 for v in (a_row, b_row, a_row + pad, b_row + pad))
     plan = (ctypes.c_int * 4)()
-    check(L.ptmi_gemm_plan(op, M, N, K, a_row + pad, b_row + pad, N + pad, int(aligned), accumulate, epilogue, plan))
+    check(L.ptmi_gemm_plan(op, M, N, K, a_row + pad, b_row + pad, N + pad, int(aligned), accumulate, epilogue,
+                           callers_stream, plan))
     return tuple(plan)
 
 

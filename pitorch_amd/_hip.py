@@ -36,6 +36,9 @@ def hip():
     H.hipEventSynchronize.argtypes = [vp]
     H.hipEventElapsedTime.argtypes = [ctypes.POINTER(ctypes.c_float), vp, vp]
     H.hipEventDestroy.argtypes = [vp]
+    H.hipStreamCreateWithFlags.argtypes = [ctypes.POINTER(vp), ctypes.c_uint]
+    H.hipStreamSynchronize.argtypes = [vp]
+    H.hipStreamDestroy.argtypes = [vp]
     H.hipStreamBeginCapture.argtypes = [vp, i]
     H.hipStreamEndCapture.argtypes = [vp, ctypes.POINTER(vp)]
     H.hipGraphInstantiate.argtypes = [ctypes.POINTER(vp), vp, vp, vp, sz]

@@ -20,14 +20,16 @@ struct HostBuffer {
     char *dev;
 };
 
+constexpr int kScratchSlots = 5;
+
 struct LibState {
     bool inited = false;
     int device = 0;
     hipStream_t stream = nullptr;
     std::vector<Resident *> residents;
     std::vector<HostBuffer> buffers;
-    float *scratch[4] = {nullptr, nullptr, nullptr, nullptr};
-    size_t scratch_cap[4] = {0, 0, 0, 0};
+    float *scratch[kScratchSlots] = {};
+    size_t scratch_cap[kScratchSlots] = {};
     int status = PTMI_OK;
     char err[512] = {0};
 };
@@ -81,7 +83,7 @@ bool lib_initialised() { return g.inited; }
 int lib_device() { return g.device; }
 
 float *scratch_buf(int slot, size_t floats) {
-    if (slot < 0 || slot >= 4) return nullptr;
+    if (slot < 0 || slot >= kScratchSlots) return nullptr;
     if (floats <= g.scratch_cap[slot]) return g.scratch[slot];
     if (g.scratch[slot]) {
         (void)hipStreamSynchronize(g.stream);
@@ -377,7 +379,7 @@ void ptmi_shutdown(void) {
     g.residents.clear();
     for (HostBuffer &b : g.buffers) (void)hipFree(b.dev);
     g.buffers.clear();
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < kScratchSlots; i++) {
         if (g.scratch[i]) (void)hipFree(g.scratch[i]);
         g.scratch[i] = nullptr;
         g.scratch_cap[i] = 0;

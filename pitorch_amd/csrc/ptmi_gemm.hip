@@ -1670,6 +1670,17 @@ size_t gemm_dev_ws_floats(int M, int N) {
     return std::min<size_t>((size_t)M * N * 64, (size_t)64 << 20);
 }
 
+// Calls on the library's stream follow one another and may all split K through
+// one workspace.  Those on streams of the caller may overlap, so they split only
+// where the fp32 tiles would (split_plan; few blocks, long K), through a
+// workspace of their own: a GEMM that those tiles run whole shares nothing
+// with a call on another stream.
+static bool callers_stream(const void *stream) { return stream && stream != (const void *)lib_stream(); }
+static size_t split_ws_floats(int op, int M, int N, int K, bool callers) {
+    const size_t n = gemm_dev_ws_floats(M, N);
+    return callers && gemm_workspace_floats(op, M, N, K, n) == 0 ? 0 : n;
+}
+
 // ── the entry point that allocates nothing ───────────────────────────────
 // ptmi_gemm_dev_noalloc keeps its split-K partials in this file-scope
 // device array (16 MiB; each GPU the library runs on holds it until the
@@ -1714,7 +1725,7 @@ int ptmi_gemm_dev_noalloc(int op, const float *dA, long lda, const float *dB, lo
     // the split is chosen from ptmi_gemm_dev's workspace size, not the
     // scratch's, so that both take the same number of splits
     return launch_gemm(op, dA, lda, dB, ldb, dC, ldc, M, N, K, accumulate, ws,
-                       std::min(kNoAllocScratchFloats, gemm_dev_ws_floats(M, N)),
+                       std::min(kNoAllocScratchFloats, split_ws_floats(op, M, N, K, callers_stream(stream))),
                        stream ? (hipStream_t)stream : lib_stream());
 }
 
@@ -1722,18 +1733,20 @@ int ptmi_gemm_dev(int op, const float *dA, long lda, const float *dB, long ldb, 
                   int K, int accumulate, void *stream) {
     int st = ensure_init();
     if (st) return st;
-    const size_t ws_n = gemm_dev_ws_floats(M, N);
-    float *ws = scratch_buf(3, ws_n);
-    if (!ws) return ptmi_last_status();
+    const bool callers = callers_stream(stream);
+    const size_t ws_n = split_ws_floats(op, M, N, K, callers);
+    float *ws = ws_n ? scratch_buf(callers ? 4 : 3, ws_n) : nullptr;
+    if (ws_n && !ws) return ptmi_last_status();
     return launch_gemm(op, dA, lda, dB, ldb, dC, ldc, M, N, K, accumulate, ws, ws_n,
                        stream ? (hipStream_t)stream : lib_stream());
 }
 
 int ptmi_gemm_plan(int op, int M, int N, int K, long lda, long ldb, long ldc, int aligned, int accumulate, int epilogue,
-                   int plan[4]) {
+                   int callers, int plan[4]) {
     if (!plan || op < 0 || op > 2 || M <= 0 || N <= 0 || K <= 0 || epilogue < GEMM_EPI_NONE || epilogue > GEMM_EPI_SWIGLU_BWD)
         return set_error(PTMI_ERR_ARG, "ptmi_gemm_plan: bad arguments");
-    const GemmChoice c = gemm_choice(op, M, N, K, lda, ldb, ldc, aligned != 0, accumulate != 0, gemm_dev_ws_floats(M, N), epilogue);
+    const GemmChoice c = gemm_choice(op, M, N, K, lda, ldb, ldc, aligned != 0, accumulate != 0,
+                                     split_ws_floats(op, M, N, K, callers != 0), epilogue);
     plan[0] = c.tm;
     plan[1] = c.tn;
     plan[2] = c.kind != GEMM_64 && c.kind != GEMM_128;

@@ -53,3 +53,24 @@ def test_plans_hold_over_the_range():
         # rows too long for the bf16 tiles' 32-bit offsets
         assert pa.gemm_plan(op, M, N, K, pad=1 << 22, accumulate=acc, epilogue=epi)[2] == 1
     assert seen == {F32, F64, DL, B64, B128}
+
+
+def test_calls_on_other_streams_share_no_workspace_they_did_not_need():
+    """K is cut on a caller's stream only where the fp32 tiles cut it: 32x32
+    tiles, fewer than 128 and K > 288, or K >= 4096 (and NT outputs of 4 Mi elements):
+    fewer than 512 tiles of 64x64."""
+    rng, cut = random.Random(4), 0
+    tiles = lambda M, N, T: -(-M // T) * -(-N // T)
+    for _ in range(6000):
+        M, N, K = (int(2 ** rng.uniform(0, e)) for e in (12, 13, 15))
+        op, acc = rng.randrange(3), rng.randrange(2)
+        splits = pa.gemm_plan(op, M, N, K, accumulate=acc, callers_stream=1)[3]
+        big = op == 2 and M * N >= 4 << 20
+        may = tiles(M, N, 64) < 512 if K >= 4096 else not big and tiles(M, N, 32) < 128 and K > 288
+        assert splits == 1 or may, (op, M, N, K)
+        cut += splits > 1
+        if may:                                          # nothing else differs from the library's stream
+            assert pa.gemm_plan(op, M, N, K, accumulate=acc, callers_stream=1) == pa.gemm_plan(op, M, N, K, accumulate=acc)
+    assert cut > 500
+    for op, M, N, K in ((0, 512, 768, 2048), (0, 300, 512, 1536)):
+        assert pa.gemm_plan(op, M, N, K)[3] > 1 and pa.gemm_plan(op, M, N, K, callers_stream=1)[3] == 1

@@ -334,6 +334,35 @@ def test_gemm_dev_short_k(op, M, N, K, acc, pad, kernel):
         d.free()
 
 
+@pytest.mark.parametrize("op,M,N,K", [(0, 512, 768, 2048), (0, 300, 512, 1536), (1, 700, 500, 1200)])
+def test_gemm_dev_on_two_streams(op, M, N, K):
+    """GEMMs on two streams of the caller and on the library's, all in flight
+    at once: each is whole on the caller's streams, cut on the library's."""
+    import ctypes
+    from pitorch_amd._hip import hip
+    L, H = pa.load_ptmi(), hip()
+    assert pa.gemm_plan(op, M, N, K)[3] > 1 and pa.gemm_plan(op, M, N, K, callers_stream=1)[3] == 1
+    assert L.ptmi_init(0) == 0
+    streams = [ctypes.c_void_p(), ctypes.c_void_p()]
+    for s in streams:
+        assert H.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0             # hipStreamNonBlocking
+    jobs = []
+    for i, s in enumerate((*streams, None)):
+        A, B = ints((K, M) if op == 1 else (M, K), 70 + i), ints((N, K) if op == 2 else (K, N), 80 + i)
+        ref = (A.T if op == 1 else A).astype(np.float64) @ (B.T if op == 2 else B).astype(np.float64)
+        jobs.append((s, A, B, DeviceArray.from_host(A), DeviceArray.from_host(B), DeviceArray(M * N), ref))
+    for _ in range(20):
+        for s, A, B, dA, dB, dC, _ref in jobs:
+            assert L.ptmi_gemm_dev(op, dA.ptr, A.shape[1], dB.ptr, B.shape[1], dC.ptr, N, M, N, K, 0, s) == 0
+    assert H.hipDeviceSynchronize() == 0
+    for s, A, B, dA, dB, dC, ref in jobs:
+        assert np.array_equal(dC.download().reshape(M, N), ref.astype(np.float32))
+        for d in (dA, dB, dC):
+            d.free()
+    for s in streams:
+        assert H.hipStreamDestroy(s) == 0
+
+
 def test_gemm_errors():
     L = pa.load_ptmi()
     A = np.ones((4, 4), np.float32)
