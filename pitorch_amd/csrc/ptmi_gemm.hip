@@ -1494,7 +1494,18 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
     g.partial = splits > 1 ? ws : nullptr;
     g.epi = epi ? *epi : GemmEpi{};
     g.nrm = norm ? *norm : GemmNorm{};
-    if ((M + 63) / 64 > 65535 || gy > 65535) return set_error(PTMI_ERR_ARG, "gemm: M too large");
+    // The grid holds 65535 tiles along M.  More rows than 65535 tiles of split_plan's are
+    // refused; where its tiles are 64 rows and the choice's 32, they go in two parts.
+    const int plan_rows = K >= 4096 || (op == 2 && (long)M * N >= (4L << 20)) ? 64 : 32;
+    if ((M + plan_rows - 1) / plan_rows > 65535) return set_error(PTMI_ERR_ARG, "gemm: M too large");
+    if (gy > 65535) {
+        if (ek != GEMM_EPI_NONE || defer) return set_error(PTMI_ERR_ARG, "gemm: M too large");
+        const int rows = 65535 * ch.tm;
+        const int st = launch_gemm(op, A, lda, B, ldb, C, ldc, rows, N, K, accumulate, ws, ws_floats, s, Cin);
+        if (st) return st;
+        return launch_gemm(op, A + (AT ? (long)rows : (long)rows * lda), lda, B, ldb, C + (long)rows * ldc, ldc, M - rows, N, K,
+                           accumulate, ws, ws_floats, s, Cin ? Cin + (long)rows * ldc : nullptr);
+    }
     dim3 grid(gx, gy, splits);
     using KFn = void (*)(GemmArgs);
     static const KFn kernels[2][3] = {

@@ -363,6 +363,21 @@ def test_gemm_dev_on_two_streams(op, M, N, K):
         assert H.hipStreamDestroy(s) == 0
 
 
+# More rows than one grid's 65535 tiles of 32: split_plan counts 64-row tiles
+# for NT outputs of 4 Mi elements, and takes 65535 of those.
+@pytest.mark.parametrize("acc", [0, 1])
+def test_gemm_dev_most_rows(acc):
+    M, N, K = 2200003, 2, 5
+    assert pa.gemm_plan(2, M, N, K, accumulate=acc)[:3] == (32, 32, 1)
+    A, B, C0 = ints((M, K), 91), ints((K, N), 92), ints((M, N), 93)
+    ref = (A @ B + (C0 if acc else 0)).astype(np.float32)
+    assert np.array_equal(split_tile_call(2, A, B, C0, M, N, K, acc, 0), ref)
+    a = DeviceArray(16)
+    assert pa.load_ptmi().ptmi_gemm_dev(2, a.ptr, K, a.ptr, K, a.ptr, N, 65535 * 64 + 1, N, K, 0, None) == 1
+    assert b"M too large" in pa.load_ptmi().ptmi_last_error()
+    a.free()
+
+
 def test_gemm_errors():
     L = pa.load_ptmi()
     A = np.ones((4, 4), np.float32)
