@@ -158,7 +158,7 @@ __device__ __forceinline__ float xmax_groups(float v) {   // over lanes l, l^16,
 }
 __device__ __forceinline__ float xsum_groups(float v) { return xsum32(xsum16(v)); }
 
-// Forward: query rows [16*QT*tile, ...) of head blockIdx.y, at positions
+// Forward: query rows [16*QT*tile, ...) of head blockIdx.x, at positions
 // pos0 + row, over keys 0..position.  The last rows (the most keys) go out
 // first, so that short blocks fill in behind the long ones.
 template <int HQ, int QT, int NW, bool PAD>

@@ -1268,7 +1268,11 @@ int enqueue_train(ptmi_model *m, int T, hipStream_t s, TrainTracer *tr = nullptr
             hipLaunchKernelGGL(mf_fwd[HQ - 1], dim3((T + kAttnRows - 1) / kAttnRows, NH), dim3(kMT), mf_lds, s, qkv, att,
                                ao, T, D, QS, scale, pitch);
         } else {
-            const AttnFwdArgs fa = {qkv, QS, qkv + D, qkv + 2 * D, QS, ao, D, row_max(l), row_inv(l), stat_ld, T, 0, hd, scale};
+            // Not the last position: no row but its own reads what it attends to, and its loss
+            // is not taken; in a tile with others its values would meet their zero weights,
+            // which an infinity or NaN turns into NaN.  (Its row stays as it was: zeros or
+            // an earlier step's.)
+            const AttnFwdArgs fa = {qkv, QS, qkv + D, qkv + 2 * D, QS, ao, D, row_max(l), row_inv(l), stat_ld, R, 0, hd, scale};
             if ((st = launch_attn_fwd(fa, NH, s))) return st;
         }
         // residual: rmid = rin + att_out . Wo^T (inside the attention span,

@@ -114,6 +114,28 @@ def untie(blob, cfg, seed):
     return np.concatenate([h.view(np.uint8), blob[28:], wcls.view(np.uint8)])
 
 
+# The last position's token is only predicted, so nothing of it may reach
+# another row: a NaN there leaves the loss and every update as the
+# reference has them (pt_train.c:224-258 sums over the keys up to the row).
+# Lengths and head sizes of the tiled attention, the last row not alone in its tile.
+@pytest.mark.parametrize("cfg,T", [((64, 160, 2, 4, 4, 512, 1024), 1024), ((256, 256, 2, 4, 4, 512, 1020), 1011),
+                                   ((72, 128, 1, 2, 2, 301, 800), 790), ((48, 128, 2, 2, 2, 400, 64), 40),
+                                   ((128, 256, 1, 1, 1, 300, 1100), 1100)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_last_position_reaches_no_other_row(cfg, T, bad):
+    blob = untie(pa.synth_model(cfg, 17, 0.05), cfg, 18)
+    tokens = pa.seed_tokens(19, T, cfg[5] - 1)
+    tokens[-1] = cfg[5] - 1
+    blob[28:].view(np.float32)[(cfg[5] - 1) * cfg[0] + 3] = bad
+    om, m = OracleModel(blob.copy(), max_T=T), pa.Model(blob, max_T=T)
+    lo, lg = om.train_step(tokens, 0.05), m.train_step(tokens, 0.05)
+    assert np.isfinite(lo) and abs(lg - lo) <= 1e-5 * abs(lo), (lg, lo)
+    w = np.frombuffer(m.read_weights().tobytes(), np.float32, offset=28)
+    assert np.array_equal(np.isfinite(w), np.isfinite(np.frombuffer(om.blob.tobytes(), np.float32, offset=28)))
+    m.close()
+    om.close()
+
+
 @pytest.mark.parametrize("untied", [False, True])
 def test_steps_with_changing_tokens_match_oracle(untied):
     """Three SGD steps over different token sequences and lengths, with the
