@@ -1198,17 +1198,30 @@ __device__ __forceinline__ void gemm_tile_slice64(const GemmArgs &g, int m0, int
 #pragma unroll
         for (int e = 0; e < T / NW; e++) sum[e] = red[(e * NW + wave) * T + lane];
     }
-    if (EPI == GEMM_EPI_NONE && !g.upd) {                       // uniform
+    if constexpr (EPI == GEMM_EPI_NONE) {
         const TileOut o(g, m0, n0, z);
         int off[T / NW];
 #pragma unroll
         for (int e = 0; e < T / NW; e++) off[e] = o.at(e * NW + wave, lane);
         o.put(sum, off);
-        return;
-    }
-    const float lrv = g.upd ? *g.lr : 0.0f;
+        if (!g.upd) return;                                     // uniform
+        // sgd_step (pt_train.c:870-873) on the weight this gradient belongs to, rows not kept
+        const float lrv = *g.lr;
+        const __amdgpu_buffer_rsrc_t upd = __builtin_amdgcn_make_buffer_rsrc(g.upd + (long)m0 * g.ldc + n0, (short)0, 0x7fffffff, 0x00020000);
+        float w[T / NW];
 #pragma unroll
-    for (int e = 0; e < T / NW; e++) store_elem<EPI>(g, sum[e], m0 + e * NW + wave, n0 + lane, z, lrv);
+        for (int e = 0; e < T / NW; e++) {
+            const int m = min(m0 + e * NW + wave, g.M - 1);
+            if (g.keep && ((g.keep[m >> 5] >> (m & 31)) & 1u)) off[e] = kOutside;
+            w[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(upd, off[e], 0, 0));
+        }
+#pragma unroll
+        for (int e = 0; e < T / NW; e++)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, w[e] - lrv * sum[e]), upd, off[e], 0, 0);
+    } else {
+#pragma unroll
+        for (int e = 0; e < T / NW; e++) store_elem<EPI>(g, sum[e], m0 + e * NW + wave, n0 + lane, z, 0.0f);
+    }
 }
 
 // Workgroups go to the 8 XCDs round-robin by linear id, and each XCD has its
@@ -1592,20 +1605,19 @@ size_t gemm_group_desc_bytes(int n) { return sizeof(GemmGroupDesc) * (size_t)n; 
 int gemm_tn_group_prepare(const TnGemm *list, int n, const float *lr, void *host_desc, TnGroupPlan *plan) {
     GemmGroupDesc *d = static_cast<GemmGroupDesc *>(host_desc);
     int vec = 1;
-    // Tile: the smaller estimate over all entries.  The 64 tiles' is
-    // gemm_choice's plus 4.4 us per tile for the weights' update, which the
-    // many 32x32 blocks hide behind each other's products.  Whole training
-    // steps with 32 / 64 tiles, us: stories110M T=256 3276 / 3649, T=512 4862 /
-    // 4852, T=1024 8470 / 7661; stories42M T=512 2316 / 2370; 252-wide, 7
-    // layers, T=700 1138 / 1115.
-    double us32 = 3.2, us64 = 4.0;
+    // Tile: the smaller estimate over all entries.  The 64 tiles' counts 3.4 us more per
+    // tile than gemm_choice's for the weights' update, which the many 32x32 blocks hide
+    // behind each other's products.  Whole training steps with 32 / 64 tiles, us:
+    // stories110M T=256 3315 / 3536, T=384 4206 / 4231, T=512 5079 / 4917, T=1024 8784 /
+    // 7870; stories42M T=512 2322 / 2307; 252-wide, 7 layers, T=400 829 / 827, T=700 1070 / 1043.
+    double us32 = 3.2, us64 = 3.6;
     bool fits = true;
     for (int i = 0; i < n; i++) {
         const TnGemm &e = list[i];
         auto blocks = [&](int T) { return (double)((e.M + T - 1) / T) * ((e.N + T - 1) / T); };
         us32 += (e.K + BK - 1) / BK * 0.19 * blocks(32) / 256.0;
-        us64 += (7.0 + 0.65 * ((e.K + 63) / 64)) * blocks(64) / 256.0;
-        fits = fits && e.lda < kMaxSplitLd && e.ldb < kMaxSplitLd;
+        us64 += (6.0 + 0.65 * ((e.K + 63) / 64)) * blocks(64) / 256.0;
+        fits = fits && std::max({e.lda, e.ldb, e.ldc}) < kMaxSplitLd;
     }
     const int tile = fits && us64 < us32 ? 64 : 32;
     int t = 0;
