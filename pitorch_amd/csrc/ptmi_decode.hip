@@ -582,7 +582,7 @@ int ptmi_model_create(const void *blob, size_t bytes, int max_T, ptmi_model_t **
         }
         memcpy(m->prefetch_plan, pp, 8);
     }
-    if ((st = decode_step_create(m)) || (st = prefill_create(m)) || (!m->eager && (st = build_graph(m))) ||
+    if ((st = decode_step_create(m)) || (!m->eager && (st = build_graph(m))) ||
         (max_T > 0 && (st = train_create(m)))) {
         train_destroy(m);
         prefill_destroy(m);
@@ -596,6 +596,7 @@ int ptmi_model_create(const void *blob, size_t bytes, int max_T, ptmi_model_t **
         release_blob(r);
         return st;
     }
+    if (max_T == 0) (void)prefill_reserve(m);            // last: it may do without
     *out = m;
     return PTMI_OK;
 }

@@ -68,7 +68,7 @@ struct ptmi_model {
     int step_n_stamps = 0;
     std::vector<int> step_cuts;          // launch windows: stages [cuts[w], cuts[w+1])
     ptmi::TrainState *train = nullptr;
-    // Prompt pass (prefill_create): rows of residual stream, normalised rows,
+    // Prompt pass (prefill_reserve): rows of residual stream, normalised rows,
     // [q | k | v] columns, attention output, hidden; split-K workspace.
     float *pre_mem = nullptr;
     float *pre_x = nullptr, *pre_xn = nullptr, *pre_q = nullptr, *pre_ao = nullptr, *pre_sh = nullptr, *pre_ws = nullptr;
@@ -86,9 +86,9 @@ void train_destroy(ptmi_model *m);
 void launch_rmsnorm_rows(float *in, const float *w, float *out, int rows, int D, const SplitK &pk, const float *cin,
                          const int *tok, const float *emb, unsigned *tok_bits, hipStream_t s);
 // The prompt's keys and values, all positions at once.
-int  prefill_create(ptmi_model *m);
+bool prefill_reserve(ptmi_model *m);
 void prefill_destroy(ptmi_model *m);
-int  prefill_positions(const ptmi_model *m, int n_prompt, int max_tokens);
+int  prefill_positions(ptmi_model *m, int n_prompt, int max_tokens);   // 0: token by token
 int  enqueue_prefill(ptmi_model *m, int n, hipStream_t s);
 // 1/pt_sqrtf(head_dim) evaluated on the host (llama2.c:137)
 float host_att_scale(int head_dim);

@@ -34,25 +34,33 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace
 
-int prefill_positions(const ptmi_model *m, int n_prompt, int max_tokens) {
-    // the last position run is a decode step: its logits are the call's
-    const int n = std::min(n_prompt, max_tokens) - 1;
-    return n >= kMinPrefill ? n : 0;
-}
-
-int prefill_create(ptmi_model *m) {
+// The pass's buffers (stories110M: 59 MB), once per model: at creation for a
+// model that does not train, else with the first prompt that needs them.
+// Without room for them the prompt runs token by token.
+bool prefill_reserve(ptmi_model *m) {
+    if (m->pre_mem) return true;
     const Config &c = m->c;
     const size_t R = std::min(c.seq_len, kPrefillRows), D = c.dim, H = c.hidden;
     size_t sizes[] = {R * D, R * D, R * 3 * D, R * D, R * H, kPrefillWs};
     float **dst[] = {&m->pre_x, &m->pre_xn, &m->pre_q, &m->pre_ao, &m->pre_sh, &m->pre_ws};
     size_t total = 0;
     for (size_t n : sizes) total += align_up(n, 64);
-    PTMI_HIP(hipMalloc(&m->pre_mem, total * sizeof(float)));
+    if (hipMalloc(&m->pre_mem, total * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        m->pre_mem = nullptr;
+        return false;
+    }
     size_t o = 0;
     for (int i = 0; i < 6; i++) { *dst[i] = m->pre_mem + o; o += align_up(sizes[i], 64); }
     m->pre_rows = (int)R;
     m->pre_ws_floats = kPrefillWs;
-    return PTMI_OK;
+    return true;
+}
+
+int prefill_positions(ptmi_model *m, int n_prompt, int max_tokens) {
+    // the last position run is a decode step: its logits are the call's
+    const int n = std::min(n_prompt, max_tokens) - 1;
+    return n >= kMinPrefill && prefill_reserve(m) ? n : 0;
 }
 
 void prefill_destroy(ptmi_model *m) {

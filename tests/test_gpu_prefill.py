@@ -56,3 +56,32 @@ def test_prompt_pass_matches_oracle(cfg, n_prompt, total):
     m2.close()
     m.close()
     om.close()
+
+
+def device_bytes_free():
+    import ctypes
+    from pitorch_amd._hip import hip
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_training_model_reserves_the_buffers_with_its_first_prompt():
+    """A model that trains holds the prompt pass's buffers (here 8 Mi floats of
+    split-K sums and 1024 rows) only once a prompt needs them."""
+    cfg = (256, 512, 1, 4, 4, 512, 1024)
+    blob = pa.synth_model(cfg, 23)
+    m, m2 = pa.Model(blob, max_T=16), pa.Model(blob)
+    prompt = np.array(pa.seed_tokens(4, 40, cfg[5]), np.int32)
+    m.generate(prompt[:4], 8, stop_on_eos=False)
+    before = device_bytes_free()
+    got = m.generate(prompt, 48, stop_on_eos=False)
+    held = before - device_bytes_free()
+    assert held >= 4 * ((8 << 20) + 1024 * (6 * 256 + 512)) // 2
+    assert list(got) == list(m2.generate(prompt, 48, stop_on_eos=False)) and np.array_equal(m.logits(), m2.logits())
+    before = device_bytes_free()
+    m2.generate(prompt, 48, stop_on_eos=False)
+    m.generate(prompt, 48, stop_on_eos=False)
+    assert before == device_bytes_free()
+    m.close()
+    m2.close()
