@@ -1424,7 +1424,8 @@ GemmChoice gemm_choice(int op, int M, int N, int K, long lda, long ldb, long ldc
         for (int T = 64; T <= 128; T += 64) {
             if (kps > (T == 64 ? 4 : 1) * p.k_per_split) continue;
             const double n = blocks(T) * splits / cus;
-            if (T == 128 && n < 1.0) continue;
+            // (RoPE's N is 3K: there 128x128 would lead, by 5%, only from 2048 rows of 2048-wide models)
+            if (T == 128 && (n < 1.0 || ek == GEMM_EPI_ROPE)) continue;
             const double per = T == 64 ? 1.85 + 0.65 * std::max(2.0, steps(kps, 64)) : 2.8 + (n > 1.0 ? 1.3 : 2.0) * steps(kps, BK);
             const double us = (T == 64 ? 3.6 : 3.2) + (vec ? 1.0 : 1.2) * std::ceil(n) * per + red;
             if (us < best.us)
@@ -1556,7 +1557,7 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
         static const KFn fused[2][3] = {                 // by epilogue kind - 1
             {k_gemm_split<false, false, 64, 4, GEMM_EPI_ROPE>, k_gemm_split<false, false, 64, 4, GEMM_EPI_SWIGLU>,
              k_gemm_split<false, true, 64, 4, GEMM_EPI_SWIGLU_BWD>},
-            {k_gemm_split<false, false, 128, 4, GEMM_EPI_ROPE>, k_gemm_split<false, false, 128, 4, GEMM_EPI_SWIGLU>,
+            {nullptr, k_gemm_split<false, false, 128, 4, GEMM_EPI_SWIGLU>,
              k_gemm_split<false, true, 128, 4, GEMM_EPI_SWIGLU_BWD>}};
         const int big = ch.kind == GEMM_128;
         fn = ek != GEMM_EPI_NONE ? fused[big][ek - 1] : plain[big][vec][op];

@@ -19,7 +19,15 @@ PADDED_HEAD = (108, 260, 2, 3, 3, 512, 160)      # head_dim 36: no multiple of 1
 WIDE_HEAD = (256, 512, 2, 2, 2, 512, 96)         # head_dim 128
 ONE_LAYER = (96, 256, 1, 3, 3, 512, 96)          # keys and values only
 WIDE = (2304, 260, 1, 24, 24, 512, 48)           # norm rows past one wave's registers
+SPLIT_TILES = (768, 1280, 2, 12, 12, 512, 640)   # its long prompts' GEMMs run on the bf16-product tiles
 TWO_PASSES = (32, 64, 2, 2, 2, 512, 1200)        # more positions than one pass takes
+
+
+def test_long_prompts_take_the_split_tiles():
+    D, H = SPLIT_TILES[:2]
+    for n in (601, 617):
+        for N, K, epi in ((3 * D, D, 1), (2 * D, D, 1), (2 * H, D, 2), (D, D, 0), (D, H, 0)):
+            assert pa.gemm_plan(2, n, N, K, epilogue=epi, accumulate=not epi)[:3] == (64, 64, 0), (n, N, K)
 
 
 @pytest.mark.parametrize("cfg,n_prompt,total", [
@@ -29,6 +37,7 @@ TWO_PASSES = (32, 64, 2, 2, 2, 512, 1200)        # more positions than one pass 
     *[(WIDE_HEAD, n, n + 2) for n in (6, 50, 90)],
     *[(ONE_LAYER, n, n + 2) for n in (6, 70)],
     *[(WIDE, n, n + 2) for n in (6, 40)],
+    *[(SPLIT_TILES, n, n + 2) for n in (602, 618)],
     *[(TWO_PASSES, n, n + 2) for n in (1024, 1025, 1026, 1031, 1190)],
 ])
 def test_prompt_pass_matches_oracle(cfg, n_prompt, total):

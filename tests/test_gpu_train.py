@@ -49,6 +49,19 @@ def test_one_step_matches_oracle(cfg, T):
     check_one_step(cfg, T)
 
 
+# The fused RoPE, SwiGLU and SwiGLU-backward epilogues on the bf16-product
+# tiles (64x64 at stories110M's width; 128x128 for a wide feed-forward), and the
+# weight gradients' 64x64 tiles, all with ragged rows.
+@pytest.mark.parametrize("cfg,T,swiglu", [((768, 1280, 1, 12, 12, 300, 640), 617, 64), ((128, 2304, 1, 2, 2, 300, 2048), 2045, 128)])
+def test_wide_step_matches_oracle(cfg, T, swiglu):
+    D, H = cfg[:2]
+    if swiglu == 64:
+        assert pa.gemm_plan(2, T, 3 * D, D, epilogue=1)[:3] == (64, 64, 0)
+    assert pa.gemm_plan(2, T, 2 * H, D, epilogue=2)[:3] == (swiglu, swiglu, 0)
+    assert pa.gemm_plan(0, T - 1, H, D, epilogue=3)[:3] == (swiglu, swiglu, 0)
+    check_one_step(cfg, T)
+
+
 # The forward RMSNorms run inside the next GEMM's A loads when it can take
 # them (GemmNorm kinds: 1 the row itself, 2 the pending split-K partials
 # plus the residual, 4 the embedding gather; default 1|4).  Every choice is
