@@ -172,8 +172,9 @@ int ptmi_gemm_plan(int op, int M, int N, int K, long lda, long ldb, long ldc,
  * split-K partial sums go to a fixed 16 MiB device scratch array that the
  * library holds on each GPU for the life of the process, located once by
  * ptmi_init (which must have been called: PTMI_ERR_STATE otherwise).  A
- * GEMM whose K split needs more than 4 Mi floats of partials (splits*M*N)
- * is rejected with PTMI_ERR_ARG before anything is enqueued.  Every call
+ * GEMM whose K the fp32 tiles would cut into pieces of more than 4 Mi floats
+ * in all (pieces*M*N, counted before the kernel is chosen) is rejected with
+ * PTMI_ERR_ARG before anything is enqueued.  Every call
  * on a GPU shares that GPU's scratch: calls that can overlap on one GPU
  * (other streams, other threads) race.  Nothing needs clearing between
  * calls: each launch writes every partial it later reads.              */

@@ -1,5 +1,5 @@
 // fp32 GEMMs on the CDNA4 matrix cores: C[M,N] (+)= op(A)[M,K] . op(B)[K,N],
-// small ones with v_mfma_f32_16x16x4_f32, the others as exact three-way bf16
+// small ones with v_mfma_f32_16x16x4_f32, the others as products of three-way bf16
 // splits with v_mfma_f32_32x32x16_bf16 (gemm_choice).  These replace the training backward's
 // per-position matvecs / CPU outer products:
 //   dW = dY^T X  (TN) — matmul_backward_weight_batched, pt_train.c:475-492
@@ -63,8 +63,8 @@ struct GemmGroupDesc {
 // the K tail), so every load is unconditional and needs no select after it.
 __device__ __align__(16) float g_gemm_zero[16] = {};
 
-// One operand tile (R rows of the M or N side x 32 k) per K step; each of
-// the 256 threads moves E = R*32/256 floats (8 or 4).  KMAJOR: the operand
+// One operand tile (R = 32 or 64 rows of the M or N side x 32 k) per K step;
+// each of the 256 threads moves E = R*32/256 floats (4 or 8).  KMAJOR (R = 32): the operand
 // is stored with k as the row index (A^T for TN, B for NN/TN); otherwise k
 // is the contiguous index.
 //   KMAJOR:  thread -> (k = tid/(R/E),     idx = E*(tid%(R/E)) + c)
@@ -115,8 +115,7 @@ __device__ __forceinline__ void load_tile(const float *P, long ld, int idx_lim, 
 }
 
 // LDS holds each operand tile k-major, S[k][col] with rows of R floats, the
-// column XOR-swizzled by row (and, for 64-wide k-major tiles, by column
-// half) so that, with LDS's 32 banks and a wave64 b32 access served as two
+// column XOR-swizzled by row so that, with LDS's 32 banks and a wave64 b32 access served as two
 // half-waves (b128 as four 8-lane groups), every access below is
 // conflict-free:
 //  * the MFMA operand reads (a half-wave reads rows k, k+1 at 16 columns):
@@ -124,14 +123,12 @@ __device__ __forceinline__ void load_tile(const float *P, long ld, int idx_lim, 
 //  * the transposing b32 stores of !KMAJOR operands (a half-wave writes one
 //    row per k group at 8 or 4 consecutive columns): the swizzle's bits
 //    3..4 (R = 64) or 2..4 (R = 32) take a different value per k group;
-//  * the b128 stores of KMAJOR operands (8 lanes write one row, 4 floats
-//    each, at a stride of E floats): for R = 64 the upper column half
-//    moves by 4 banks.
+//  * the b128 stores of KMAJOR operands (8 lanes write one row, 4 floats each).
 // Bits 0..1 are never swizzled, so float4 chunks stay whole.
 template <bool KMAJOR, int R>
 __device__ __forceinline__ int lds_col(int r, int c) {
     if constexpr (KMAJOR) {
-        if constexpr (R == 64) return c ^ ((r & 1) << 4) ^ (((c >> 5) & 1) << 2);
+        static_assert(R == 32, "k-major tiles are 32 wide");
         return c ^ ((r & 1) << 4);
     } else if constexpr (R == 64) {
         return c ^ ((((r & 1) ^ ((r >> 3) & 1)) << 4) | (((r >> 4) & 1) << 3));
@@ -470,38 +467,26 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, int m0, int n0, int
     }
 }
 
-// ── Direct-to-LDS tiles for the large training GEMMs ─────────────────────
+// ── Direct-to-LDS tiles ──────────────────────────────────────────────────
 // gfx950's global_load_lds_dwordx4 moves a 16-byte chunk per lane from
 // global memory straight into LDS, at the wave's LDS base + 16*lane (lane
-// layout checked on the MI355X).  No staging registers and no LDS store
-// instructions, so 128- and 256-row tiles fit with two waves per SIMD.
-// Each operand tile keeps its global layout in LDS, permuted in whole
+// layout checked on the MI355X): no staging registers and no LDS store
+// instructions.  Each operand tile keeps its global layout in LDS, permuted in whole
 // 16-byte chunks (the only granularity a DMA load can place):
 //  * k-contiguous operands ([i][k]: A of NN/NT, B^T of NT): rows of BK=32
 //    floats (128 bytes), chunk c of row i at slot c ^ kc_swz(i).  A lane
 //    reads the 4 k of its row for 4 MFMA steps as one b128 (lane group g
 //    takes k = 4g..4g+3 of each 16-k group).  A b128 read serves 16 lanes
 //    (16 rows) at a time across the 64 banks, where rows i and i+8 start on
-//    the same bank; kc_swz gives the 16 rows 16 distinct bank groups.  With
-//    c ^ (i & 7) alone the 32x32x2 NT tile measured 45.5% LDS conflict
-//    cycles (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE), with kc_swz 7.7%
-//    (one cycle per 64-lane b32 write of its store staging), at the same
-//    speed and bits;
+//    the same bank; kc_swz gives the 16 rows 16 distinct bank groups;
 //  * k-major operands ([k][i]: A^T of TN, B of NN/TN): rows of TI floats,
 //    the column XOR-ed with 16 in rows whose bit 2 of k is set; the two k
 //    rows a half-wave reads (g = 0, 1) then sit 16 banks apart.
 // Both operands use the same order of k inside a 16-k group (lane group g,
 // step s -> k = 4g + s), so every product pairs the same k.
-// Two LDS stages: the loads of tile s+1 are issued before the MFMAs of tile
+// The 128x96 tile below is for weight gradients (TN) of one K step (gemm_choice);
+// it has two LDS stages: the loads of tile s+1 are issued before the MFMAs of tile
 // s and waited for (vmcnt, in order) at the next step's barrier.
-// Large weight gradients (TN) over fewer than 256 positions run on these
-// tiles; longer ones and the classifier's forward (NT) take the bf16-product
-// tiles below.  Measured on the MI355X against the register-ring kernel: TN
-// 32000x288x255 with 64x96 tiles 55.5 vs 58.7 us, and with 128x96 tiles on 8
-// waves (4x2) 51.1-52.9 vs 53.6-55.1 us (graph-replayed, same output bits;
-// 128x96 on 4 or 8x1 waves, 256x96, 64x96 on 8 waves, 64x288 and 128x288 were
-// slower).  Deeper stage rings, 64-k stages, and loads interleaved one per
-// MFMA k step were all slower.
 constexpr int kDlStages = 2;
 
 // Chunk-slot swizzle of row i of a k-contiguous tile: i & 7 spreads 8
@@ -546,16 +531,14 @@ __device__ __forceinline__ void dl_issue(const float *P, long ld, int ilim, int 
     }
 }
 
-// One TMxTN output tile on WM x WN waves (each (TM/WM) x (TN/WN)).
-// AK: A stored [K][M] (TN); BKM: B stored [K][N] (NN, TN).
-template <bool AK, bool BKM, int TM, int TN, int WM, int WN, int EPI = GEMM_EPI_NONE>
+// One TMxTN output tile on WM x WN waves (each (TM/WM) x (TN/WN)), both
+// operands k-major (TN).
+template <int TM, int TN, int WM, int WN>
 __device__ __forceinline__ void gemm_tile_dl(const GemmArgs &g, int m0, int n0, int z) {
-    constexpr int NW = WM * WN, NS = kDlStages, CPI = BK / 4;
+    constexpr int NW = WM * WN, NS = kDlStages;
     constexpr int FM = TM / WM / 16, FN = TN / WN / 16;
     static_assert(FM * WM * 16 == TM && FN * WN * 16 == TN, "tile");
     constexpr int STAGE = (TM + TN) * BK;
-    constexpr int LPT = (TM * CPI / 64 + NW - 1) / NW + (TN * CPI / 64 + NW - 1) / NW;
-    static_assert((NS - 2) * LPT < 64, "vmcnt");
     __shared__ __align__(16) float smem[NS * STAGE + 256];
     float *junk = smem + NS * STAGE;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -574,41 +557,28 @@ __device__ __forceinline__ void gemm_tile_dl(const GemmArgs &g, int m0, int n0, 
     auto issue = [&](int t) {
         float *st = smem + (t % NS) * STAGE;
         const int k0 = kb + t * BK;
-        dl_issue<AK, TM, NW>(g.A, g.lda, g.M, m0, k0, kend, st, junk, wave, lane);
-        dl_issue<BKM, TN, NW>(g.B, g.ldb, g.N, n0, k0, kend, st + TM * BK, junk, wave, lane);
+        dl_issue<true, TM, NW>(g.A, g.lda, g.M, m0, k0, kend, st, junk, wave, lane);
+        dl_issue<true, TN, NW>(g.B, g.ldb, g.N, n0, k0, kend, st + TM * BK, junk, wave, lane);
     };
     // MFMA operands of 16-k group q: lane group lk takes k = 16q + 4lk + s
     // in step s (a float4 per fragment, one k per component).
     auto read_a = [&](const float *st, int q, floatx4 (&a)[FM]) {
 #pragma unroll
-        for (int f = 0; f < FM; f++) {
-            const int i = wm * (TM / WM) + f * 16 + li;
-            if constexpr (AK) {
+        for (int f = 0; f < FM; f++)
 #pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    const int k = 16 * q + 4 * lk + s;
-                    a[f][s] = st[k * TM + (i ^ (((k >> 2) & 1) << 4))];
-                }
-            } else {
-                a[f] = *reinterpret_cast<const floatx4 *>(st + (i * CPI + ((4 * q + lk) ^ kc_swz(i))) * 4);
+            for (int s = 0; s < 4; s++) {
+                const int k = 16 * q + 4 * lk + s, i = wm * (TM / WM) + f * 16 + li;
+                a[f][s] = st[k * TM + (i ^ (((k >> 2) & 1) << 4))];
             }
-        }
     };
     auto read_b = [&](const float *st, int q, floatx4 (&b)[FN]) {
-        const float *sb = st + TM * BK;
 #pragma unroll
-        for (int h = 0; h < FN; h++) {
-            const int i = wn * (TN / WN) + h * 16 + li;
-            if constexpr (BKM) {
+        for (int h = 0; h < FN; h++)
 #pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    const int k = 16 * q + 4 * lk + s;
-                    b[h][s] = sb[k * TN + (i ^ (((k >> 2) & 1) << 4))];
-                }
-            } else {
-                b[h] = *reinterpret_cast<const floatx4 *>(sb + (i * CPI + ((4 * q + lk) ^ kc_swz(i))) * 4);
+            for (int s = 0; s < 4; s++) {
+                const int k = 16 * q + 4 * lk + s, i = wn * (TN / WN) + h * 16 + li;
+                b[h][s] = st[TM * BK + k * TN + (i ^ (((k >> 2) & 1) << 4))];
             }
-        }
     };
 
     if (nk > 0) issue(0);
@@ -637,7 +607,7 @@ __device__ __forceinline__ void gemm_tile_dl(const GemmArgs &g, int m0, int n0, 
                     for (int h = 0; h < FN; h++)
                         acc[f][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][f][ss], b[q][h][ss], acc[f][h], 0, 0, 0);
     }
-    gemm_store<EPI, FM, FN>(g, acc, m0 + wm * (TM / WM), n0 + wn * (TN / WN), z, li, lk);
+    gemm_store<GEMM_EPI_NONE, FM, FN>(g, acc, m0 + wm * (TM / WM), n0 + wn * (TN / WN), z, li, lk);
 }
 
 // f(integral_constant<int, s>) for s = S...
@@ -733,8 +703,8 @@ __device__ __forceinline__ void gemm_tile_panel(const GemmArgs &g, int m0, int n
 // give it, where a sum is not finite (infinities, NaNs, numbers that round past
 // the bf16 range) or subnormal, or where an operand has bits below bf16's
 // smallest number, 2^-133, as operands below 2^-109 can.  Rounding m and
-// watching for such bits cost about 1.5% in 64x64 tiles and 0 to 6% in 128x128 ones
-// (NT 1024x32000x768 271 -> 289 us).
+// watching for such bits cost 1 to 6% (NN 1024x768x32000 283 -> 299 us, NT 1024x32000x768
+// 271 -> 289).
 // What bounds it: the MFMAs (32 cycles each) and the splits (8 VALU
 // instructions per MFMA) issue side by side; with the splits taken out the same
 // kernels reach 180-195 TFLOP/s, the bf16 matrix rate under the card's power limit.
@@ -1257,7 +1227,7 @@ __global__ __launch_bounds__(256, AT ? 1 : 2) void k_gemm(GemmArgs g) {
 }
 
 // The direct-to-LDS GEMM (grid and tile order as k_gemm).
-template <bool AK, bool BKM, int TM, int TN, int WM, int WN>
+template <int TM, int TN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void k_gemm_dl(GemmArgs g) {
     const int gx = gridDim.x, gy = gridDim.y, per_z = gx * gy, total = per_z * gridDim.z;
     int m = blockIdx.y, n = blockIdx.x, z = blockIdx.z;
@@ -1268,7 +1238,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_dl(GemmArgs g) {
         if (g.M > g.N) m = u / gx, n = u - m * gx;
         else n = u / gy, m = u - n * gy;
     }
-    gemm_tile_dl<AK, BKM, TM, TN, WM, WN>(g, m * TM, n * TN, z);
+    gemm_tile_dl<TM, TN, WM, WN>(g, m * TM, n * TN, z);
 }
 
 // The per-layer panel GEMM (grid, tile order and register bound as k_gemm).
@@ -1587,7 +1557,7 @@ int launch_gemm(int op, const float *A, long lda, const float *B, long ldb, floa
         if (pf) fn = pf;
     }
     if (ch.kind == GEMM_64F) fn = vec ? k_gemm<false, true, 64, 64, kRing32, true> : k_gemm<false, true, 64, 64, kRing32, false>;
-    if (ch.kind == GEMM_DL) fn = k_gemm_dl<true, true, 128, 96, 4, 2>;
+    if (ch.kind == GEMM_DL) fn = k_gemm_dl<128, 96, 4, 2>;
     hipLaunchKernelGGL(fn, grid, dim3(ch.kind == GEMM_DL ? 512 : 256), 0, s, g);
     PTMI_HIP(hipGetLastError());
     if (splits > 1 && defer) {
@@ -1738,13 +1708,13 @@ int ptmi_gemm_dev_noalloc(int op, const float *dA, long lda, const float *dB, lo
         return set_error(PTMI_ERR_STATE, "ptmi_gemm_dev_noalloc: call ptmi_init first (it locates the scratch)");
     float *ws = g_scratch_dev[lib_device()];
     if (!ws) return set_error(PTMI_ERR_STATE, "ptmi_gemm_dev_noalloc: no scratch on device %d", lib_device());
-    // The K split ptmi_gemm_dev would take must fit the fixed scratch, so
-    // both entries sum in the same order and give the same bits.
+    // The K split of the fp32 tiles must fit the fixed scratch, also where
+    // the bf16-product tiles (whose split always fits) take the call.
     const size_t need = gemm_workspace_floats(op, M, N, K, gemm_dev_ws_floats(M, N));
     if (need > kNoAllocScratchFloats)
         return set_error(PTMI_ERR_ARG,
-                         "ptmi_gemm_dev_noalloc: %dx%dx%d needs %zu floats of split-K partials; the fixed scratch "
-                         "holds %zu",
+                         "ptmi_gemm_dev_noalloc: %dx%dx%d counts %zu floats of split-K partials (fp32 tiles); the fixed "
+                         "scratch holds %zu",
                          M, N, K, need, kNoAllocScratchFloats);
     // the split is chosen from ptmi_gemm_dev's workspace size, not the
     // scratch's, so that both take the same number of splits

@@ -115,9 +115,8 @@ def test_backward_input_batched_exact(out_dim, in_dim):
     assert np.array_equal(dX, ref)
 
 
-# Kernel paths: 32x32 tiles (255x288x288, 300x77x130, 1x5x3, 1000x301x900),
-# 32x32 with split K (100x3001x70), 64x64 with split K (K = 32000); the
-# 64x64 NT path for large outputs runs in the 15M training-step tests.
+# Kernel paths: 32x32 tiles (255x288x288, 300x77x130, 1x5x3), 64x64 bf16-product
+# tiles (1000x301x900), the same with split K (K = 3001 and 32000).
 @pytest.mark.parametrize("M,K,N", [(255, 288, 288), (255, 32000, 288), (300, 77, 130), (1, 5, 3), (100, 3001, 70),
                                    (1000, 301, 900)])
 def test_sgemm_rect_random_bounded(M, K, N):
@@ -163,9 +162,9 @@ def test_gemm_dev_ops_with_strides(op):
 
 
 # Grids of 768 blocks and more take their tiles in XCD order (each XCD a
-# contiguous tile range, ordered along the larger operand): ragged M, N and
-# K on 64x64 and 32x32 tiles, split K for the NN forms; a NaN-filled C shows
-# any tile left unwritten.
+# contiguous tile range, ordered along the larger operand), the bf16-product
+# tiles' always do: ragged M, N and K on 64x64 and 128x128 tiles, split K for the
+# NN forms; a NaN-filled C shows any tile left unwritten.
 @pytest.mark.parametrize("op,M,N,K", [(2, 200, 20000, 300), (2, 260, 20000, 300), (0, 255, 320, 30000),
                                       (0, 130, 288, 30000), (1, 30004, 288, 130), (1, 32000, 256, 131)])
 def test_gemm_dev_large_grids(op, M, N, K):
@@ -192,9 +191,9 @@ def test_gemm_dev_large_grids(op, M, N, K):
         a.free()
 
 
-# The largest outputs (4M elements and more: NT on the bf16-product tiles, TN
-# with K < 256 on the direct-to-LDS fp32 tiles): integer-exact at the classifier shapes of config 5, with and without
-# accumulate, and on ragged M, N and K.
+# The largest outputs (4M elements and more), NT and TN: on 128x128 bf16-product
+# tiles, and on the direct-to-LDS fp32 tiles (TN, K = 7): integer-exact at the
+# classifier shapes of config 5, with and without accumulate, and on ragged M, N and K.
 @pytest.mark.parametrize("op,M,N,K,acc", [(2, 256, 32000, 288, 0), (2, 256, 32000, 288, 1), (2, 193, 21845, 36, 1),
                                           (1, 32000, 288, 255, 0), (1, 32000, 288, 255, 1), (1, 16388, 260, 7, 0)])
 def test_gemm_dev_direct_lds_exact(op, M, N, K, acc):
@@ -239,10 +238,10 @@ def test_gemm_dev_panel_nt_exact(M, N, K, acc):
         a.free()
 
 
-# The bf16-product tiles (middle and large GEMMs: 64x64 with K dealt to four
-# waves, 128x128 for many tiles): every op, whole and ragged M, N and K, K ranges
-# that leave a wave without work, split K, rows without 16-byte alignment,
-# padded leading dimensions, accumulate.
+# Middle and large GEMMs, mostly on the bf16-product tiles (64x64 with K dealt to
+# four waves, 128x128 for many tiles; tests/test_gpu_gemm_split.py holds each of
+# them): whole and ragged M, N and K, K ranges that leave a wave without work,
+# split K, rows without 16-byte alignment, padded leading dimensions, accumulate.
 SPLIT_TILES = [(0, 1024, 768, 2048, 0, 0), (1, 770, 2050, 1000, 1, 2), (2, 1024, 2048, 768, 1, 0), (2, 333, 8001, 701, 0, 0),
                (0, 501, 517, 1003, 1, 0), (1, 1003, 517, 501, 0, 1), (0, 65, 4100, 4097, 0, 3), (2, 200, 32000, 300, 1, 0),
                (1, 33000, 130, 300, 0, 0), (2, 257, 21847, 37, 0, 0), (0, 700, 12000, 260, 0, 4), (2, 64, 65600, 20, 0, 0)]
