@@ -334,6 +334,10 @@ __device__ __forceinline__ floatx4 load4_any(const float *p) { return *reinterpr
 __device__ __forceinline__ floatx4 stream4_any(const float *p) {
     return __builtin_nontemporal_load(reinterpret_cast<const floatx4_any *>(p));
 }
+template <bool NT>
+__device__ __forceinline__ floatx4 weight4_any(const float *p) {
+    return NT ? stream4_any(p) : load4_any(p);
+}
 __device__ __forceinline__ floatx4 keep4(bool keep, floatx4 v) {
     return floatx4{keep ? v.x : 0.0f, keep ? v.y : 0.0f, keep ? v.z : 0.0f, keep ? v.w : 0.0f};
 }
@@ -350,9 +354,9 @@ __device__ __forceinline__ void store_row(const MatvecParams &p, long r, float v
 // Long rows: a block of W waves takes RB rows, its waves interleaved passes of 4
 // float4 per lane and row, so a few hundred rows already fill the chip (one
 // wave per row pair kept 384 waves with one load pair each in flight on 768
-// rows).  Measured: 768x32000 (the transposed classifier) 66 -> 18 us (5.4 TB/s;
-// a lone launch reaches 6.0), 288x32000 9.7, 2048x4096 7.0, 4000x8003 21.7.
-template <int W, int RB>
+// rows).  NT: the weights pass by the caches.  Measured: 768x32000 (the transposed
+// classifier) 66 -> 18 us (5.4 TB/s; a lone launch reaches 6.0), 288x32000 9.7.
+template <int W, int RB, bool NT>
 __global__ __launch_bounds__(64 * W) void k_matvec_long(MatvecParams p) {
     constexpr int U = 4;
     __shared__ float part[W][RB];
@@ -371,7 +375,7 @@ __global__ __launch_bounds__(64 * W) void k_matvec_long(MatvecParams p) {
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int r = 0; r < RB; r++) wv[r][u] = stream4_any(w[r] + 4L * min(c0 + 64 * u, n4 - 1));
+            for (int r = 0; r < RB; r++) wv[r][u] = weight4_any<NT>(w[r] + 4L * min(c0 + 64 * u, n4 - 1));
 #pragma unroll
         for (int u = 0; u < U; u++) xv[u] = load4_any(p.x + 4L * min(c0 + 64 * u, n4 - 1));
 #pragma unroll
@@ -706,13 +710,17 @@ int launch_matvec(MatvecParams p, hipStream_t s, hipEvent_t e0, hipEvent_t e1, b
         return set_error(PTMI_ERR_ARG, "matvec: fused variants need 16-byte aligned rows, n%%4==0");
     }
     if (p.n > 64 * 9 * 4) {
-        // Two rows per block share their x, unless one row each leaves less
-        // on the fullest of the 256 CUs (768 rows: 3 against 4 rows, 18.0 against
-        // 19.0 us; 288 rows: 2 and 2, 11.3 against 9.7).  Eight waves where a
-        // row gives each of them a whole pass.
-        const bool two = (((long)p.rows + 1) / 2 + 255) / 256 * 2 <= ((long)p.rows + 255) / 256;
+        // From 8192 floats a row gives each of eight waves a whole pass: two rows per
+        // block share their x, unless one row each leaves less on the fullest of the
+        // 256 CUs (768 rows: 3 against 4 rows, 18.0 against 19.0 us; 288 rows: 2 and
+        // 2, 11.3 against 9.7).  Shorter rows: four waves, one row, and loads that leave the
+        // weights in the caches, which repeated calls then read (past the caches, two
+        // rows or one: 1536x2560 4.5 -> 3.2 us, 2048x3072 5.7 -> 3.8, 3712x5344
+        // 14.6 -> 12.8; over 104 shapes 1.22 times as fast).  On weights that no cache
+        // holds the two are level (3712x5344 15.2 -> 15.6, 288x7136 4.6 -> 4.5; each 0.89 to 1.20).
         const bool eight = p.n >= 8192;
-        fn = eight ? (two ? k_matvec_long<8, 2> : k_matvec_long<8, 1>) : (two ? k_matvec_long<4, 2> : k_matvec_long<4, 1>);
+        const bool two = eight && (((long)p.rows + 1) / 2 + 255) / 256 * 2 <= ((long)p.rows + 255) / 256;
+        fn = !eight ? k_matvec_long<4, 1, false> : two ? k_matvec_long<8, 2, true> : k_matvec_long<8, 1, true>;
         const long blocks = two ? ((long)p.rows + 1) / 2 : p.rows;
         launch_k(fn, dim3((unsigned)blocks), dim3(eight ? 512 : 256), 0, s, e0, e1, p);
     } else {

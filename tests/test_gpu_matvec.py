@@ -97,6 +97,13 @@ def test_any_row_length_stride_and_start(d, n, pad, start):
         a.free()
 
 
+# Rows of the four-wave kernel (2305 to 8191 floats): parts of a last pass, one row to some thousands.
+@pytest.mark.parametrize("d,n,pad,start", [(1, 8191, 0, 0), (1366, 3072, 0, 0), (1820, 2305, 3, 1), (2049, 4097, 1, 3),
+                                           (3713, 2308, 0, 0), (513, 8188, 0, 1)])
+def test_rows_of_the_four_wave_kernel(d, n, pad, start):
+    test_any_row_length_stride_and_start(d, n, pad, start)
+
+
 def test_bad_arguments_are_errors():
     L = pa.load_ptmi()
     W = np.ones((4, 4), np.float32)
