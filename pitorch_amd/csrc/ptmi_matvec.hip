@@ -408,9 +408,10 @@ __global__ __launch_bounds__(64 * W) void k_matvec_long(MatvecParams p) {
 
 // Rows of at most 64*9*4 floats at any alignment: RW rows per wave, IT float4 of
 // each per lane (IT = ceil(n/4 / 64), 0 where n < 4), everything loaded before
-// any of it is used.  5003x1027 with 4-byte loads one after another: 7.1 us, now 5.1
-// (4.0 TB/s); 30001x301 7.8, 20001x101 4.1.
-template <int IT, int RW>
+// any of it is used.  NT: the weights pass by the caches.  5003x1027 with 4-byte
+// loads one after another: 7.1 us through the entry point, now 4.6; 30001x301 7.8,
+// 20001x101 4.1.
+template <int IT, int RW, bool NT>
 __global__ __launch_bounds__(256) void k_matvec_any(MatvecParams p) {
     const int lane = threadIdx.x & 63, n4 = p.n >> 2, tail = p.n & 3;
     const long r0 = ((long)blockIdx.x * kWaves + (threadIdx.x >> 6)) * RW;
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(256) void k_matvec_any(MatvecParams p) {
     for (int r = 0; r < RW; r++) {
         const float *w = p.W + min(r0 + r, (long)p.rows - 1) * p.ld;
 #pragma unroll
-        for (int i = 0; i < IT; i++) wv[r][i] = stream4_any(w + 4 * min(i * 64 + lane, n4 - 1));
+        for (int i = 0; i < IT; i++) wv[r][i] = weight4_any<NT>(w + 4 * min(i * 64 + lane, n4 - 1));
         wt[r] = w[jt];
     }
 #pragma unroll
@@ -501,19 +502,19 @@ KernelFn pick_xr(int it, int np) {
     return np == 2 ? pick_xr_np<LPR, 2>(it) : pick_xr_np<LPR, 1>(it);
 }
 
-template <int RW>
+template <int RW, bool NT>
 KernelFn pick_any(int it) {
     switch (it) {
-    case 0: return k_matvec_any<0, RW>;
-    case 1: return k_matvec_any<1, RW>;
-    case 2: return k_matvec_any<2, RW>;
-    case 3: return k_matvec_any<3, RW>;
-    case 4: return k_matvec_any<4, RW>;
-    case 5: return k_matvec_any<5, RW>;
-    case 6: return k_matvec_any<6, RW>;
-    case 7: return k_matvec_any<7, RW>;
-    case 8: return k_matvec_any<8, RW>;
-    default: return k_matvec_any<9, RW>;
+    case 0: return k_matvec_any<0, RW, NT>;
+    case 1: return k_matvec_any<1, RW, NT>;
+    case 2: return k_matvec_any<2, RW, NT>;
+    case 3: return k_matvec_any<3, RW, NT>;
+    case 4: return k_matvec_any<4, RW, NT>;
+    case 5: return k_matvec_any<5, RW, NT>;
+    case 6: return k_matvec_any<6, RW, NT>;
+    case 7: return k_matvec_any<7, RW, NT>;
+    case 8: return k_matvec_any<8, RW, NT>;
+    default: return k_matvec_any<9, RW, NT>;
     }
 }
 
@@ -728,7 +729,12 @@ int launch_matvec(MatvecParams p, hipStream_t s, hipEvent_t e0, hipEvent_t e1, b
         // rows, whose loads leave registers for it) four
         const int it = (p.n / 4 + 63) / 64;
         const int rw = p.rows <= kBigWaves ? 1 : p.rows <= 2 * kBigWaves || it > 4 ? 2 : 4;
-        fn = rw == 1 ? pick_any<1>(it) : rw == 2 ? pick_any<2>(it) : pick_any<4>(it);
+        // weights of up to 32 MB stay in the 8 x 4 MB of L2, which repeated calls then read
+        // (8192x517 4.8 -> 3.5 us, 5003x1027 4.9 -> 3.2, 12000x517 5.5 -> 4.0); past
+        // that they mostly push each other out (24000x909 13.3 -> 13.9)
+        const bool stay = (long)p.rows * p.n <= (8L << 20);
+        if (stay) fn = rw == 1 ? pick_any<1, false>(it) : rw == 2 ? pick_any<2, false>(it) : pick_any<4, false>(it);
+        else fn = rw == 1 ? pick_any<1, true>(it) : rw == 2 ? pick_any<2, true>(it) : pick_any<4, true>(it);
         const long per = (long)kWaves * rw, blocks = (p.rows + per - 1) / per;
         launch_k(fn, dim3((unsigned)blocks), dim3(kWaves * 64), 0, s, e0, e1, p);
     }

@@ -104,6 +104,13 @@ def test_rows_of_the_four_wave_kernel(d, n, pad, start):
     test_any_row_length_stride_and_start(d, n, pad, start)
 
 
+# Rows at any alignment on both sides of 8 Mi floats (the weights' loads change), one, two and four rows a wave.
+@pytest.mark.parametrize("d,n,pad,start", [(8191, 1023, 0, 1), (8192, 1025, 1, 0), (8195, 1021, 0, 0), (8213, 1023, 0, 3),
+                                           (16385, 510, 0, 2), (16449, 511, 2, 1)])
+def test_unaligned_rows_around_the_cache_rule(d, n, pad, start):
+    test_any_row_length_stride_and_start(d, n, pad, start)
+
+
 def test_bad_arguments_are_errors():
     L = pa.load_ptmi()
     W = np.ones((4, 4), np.float32)
