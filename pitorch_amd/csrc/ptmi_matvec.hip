@@ -409,8 +409,7 @@ __global__ __launch_bounds__(64 * W) void k_matvec_long(MatvecParams p) {
 // Rows of at most 64*9*4 floats at any alignment: RW rows per wave, IT float4 of
 // each per lane (IT = ceil(n/4 / 64), 0 where n < 4), everything loaded before
 // any of it is used.  NT: the weights pass by the caches.  5003x1027 with 4-byte
-// loads one after another: 7.1 us through the entry point, now 4.6; 30001x301 7.8,
-// 20001x101 4.1.
+// loads one after another: 7.1 us a call, now 3.5 (3.2 on the card); 30001x301 7.8.
 template <int IT, int RW, bool NT>
 __global__ __launch_bounds__(256) void k_matvec_any(MatvecParams p) {
     const int lane = threadIdx.x & 63, n4 = p.n >> 2, tail = p.n & 3;
